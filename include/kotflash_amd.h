@@ -217,6 +217,16 @@ int kf_kv_append(void* k_cache, void* v_cache, const void* new_k, const void* ne
                  const int64_t* new_v_strides4, int dtype, void* stream);
 
 /*
+ * Host lengths into a ragged cache's device arrays: starts[i] (int64) =
+ * seqlens[i] (int32) = lengths[i] for i < count. The values travel as kernel
+ * arguments: the call copies nothing from host memory on the stream and does
+ * not wait; `lengths` may be reused when it returns. No counterpart in the
+ * reference, whose cache has one scalar length.
+ */
+int kf_store_lengths(int64_t* starts, int32_t* seqlens, const int32_t* lengths, int64_t count,
+                     void* stream);
+
+/*
  * Fused append + split-KV decode in one decode launch (plus the merge):
  * new tokens new_k/new_v [B, Hkv, Snew, D] are stored at cache positions
  * start_b .. start_b + Snew - 1, and query rows of batch entry b attend,

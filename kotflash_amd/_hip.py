@@ -54,6 +54,7 @@ _SIGNATURES = {
                                     _I64P, _I64P, _I64P, _I64P, _F, _I, _I, _P]),
     "kf_kv_append": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
                           _I64P, _I64P, _I64P, _I64P, _I, _P]),
+    "kf_store_lengths": (_I, [_P, _P, ctypes.POINTER(ctypes.c_int32), _I64, _P]),
     "kf_attn_append_decode": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                    _I64, _I64, _I64, _I64, _I64P, _I64P, _I64P, _I64P, _I64P,
                                    _I64P, _F, _I, _I, _P, _SZ, _P]),
@@ -78,7 +79,42 @@ def lib() -> ctypes.CDLL:
     version = handle.kf_abi_version()
     if version != ABI_VERSION:
         raise RuntimeError(f"kotflash_amd ABI mismatch: library {version}, bindings {ABI_VERSION}")
+    try:
+        from . import _native  # noqa: F401
+    except ImportError as exc:
+        raise RuntimeError(f"kotflash_amd native module not usable ({exc}); build it with "
+                           "`python -m kotflash_amd.build`") from exc
     return handle
+
+
+class _NoNative:
+    """Stands in for the native module where it is not built: every call is
+    left to the Python path (which raises on a GPU, where the library is
+    missing too)."""
+
+    def __getattr__(self, name):
+        return _not_handled
+
+
+def _not_handled(*args):
+    return NotImplemented
+
+
+_NATIVE = None
+
+
+def native():
+    """``kotflash_amd._native``, the C++ launch path (csrc/native). Its entries
+    return NotImplemented, before doing anything, for calls that are not the
+    ordinary case."""
+    global _NATIVE
+    if _NATIVE is None:
+        if not library_available():
+            return _NoNative()
+        from . import _native
+
+        _NATIVE = _native
+    return _NATIVE
 
 
 def library_available() -> bool:

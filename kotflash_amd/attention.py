@@ -18,7 +18,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _hip
-from ._planning import gfx950_profile_for_shapes, t4_profile_for_shapes
+from ._planning import GFX950_HIP_MIN_FWD_FLOPS, gfx950_profile_for_shapes, t4_profile_for_shapes
 from .kernels.hip_backward import attention_backward, backward_validated
 from .kernels.hip_decode import (  # noqa: F401  strided_decode_supported: the reference's module name
     decode_supported_unchecked,
@@ -264,6 +264,12 @@ def attention(
     eager training step is host-bound and SDPA finishes first; SDPA
     everywhere else.
     """
+    # The ordinary GPU call is checked, routed and launched natively; anything
+    # else (and every error) takes the checks below.
+    if getattr(q, "is_cuda", False) and not torch.compiler.is_compiling():
+        out = _hip.native().attention(q, k, v, causal, scale, backend, GFX950_HIP_MIN_FWD_FLOPS)
+        if out is not NotImplemented:
+            return out
     _validate(q, k, v)
     if not isinstance(causal, bool):
         raise TypeError("causal must be a bool")

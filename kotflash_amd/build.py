@@ -1,4 +1,5 @@
-"""Ahead-of-time build of the gfx950 C-ABI library ``libkotflash_amd.so``.
+"""Ahead-of-time build of the gfx950 C-ABI library ``libkotflash_amd.so`` and
+of the torch-side launch path ``_native.so`` (host C++, linked against it).
 
 Each ``csrc/*.hip`` / ``csrc/*.cpp`` file is compiled by ``hipcc`` for
 ``--offload-arch=gfx950`` into ``_build/`` and linked into
@@ -15,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -24,6 +26,8 @@ BUILD_DIR = PKG_DIR / "_build"
 LIB_NAME = "libkotflash_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 ARCH = "gfx950"
+NATIVE_SRC = CSRC / "native" / "torch_binding.cpp"
+NATIVE_PATH = PKG_DIR / "_native.so"
 
 # -packed-fp32-ops: keep the compiler from forming packed fp32 VALU ops.
 HIP_FLAGS = [
@@ -81,14 +85,52 @@ def _compile(src: Path, verbose: bool) -> Path:
     return obj
 
 
+def _native_cmd(step: list[str]) -> list[str]:
+    """Host compiler command of the torch binding."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc()).resolve().parent.parent
+    includes = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include",
+                rocm / "include", Path(sysconfig.get_paths()["include"])]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *(f"-isystem{p}" for p in includes), *step, f"-L{root / 'lib'}"]
+
+
+def _run(cmd: list[str], what: str, verbose: bool) -> None:
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n" + res.stdout + res.stderr)
+
+
+def _compile_native(verbose: bool) -> Path:
+    obj = BUILD_DIR / "torch_binding.o"
+    _run(_native_cmd(["-c", str(NATIVE_SRC), "-o", str(obj)]), f"compiling {NATIVE_SRC.name}", verbose)
+    return obj
+
+
+def _link_native(obj: Path, verbose: bool) -> None:
+    tmp = NATIVE_PATH.with_suffix(".so.tmp")
+    _run(_native_cmd(["-shared", "-o", str(tmp), str(obj), f"-L{PKG_DIR}", f"-l:{LIB_NAME}"])
+         + ["-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"],
+         "native link", verbose)
+    os.replace(tmp, NATIVE_PATH)
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
-    """Compile every source and link ``libkotflash_amd.so``; returns its path."""
+    """Compile every source, link ``libkotflash_amd.so`` and the native module
+    on top of it; returns the library's path."""
     BUILD_DIR.mkdir(exist_ok=True)
     srcs = sources()
     if not srcs:
         raise RuntimeError(f"no sources under {CSRC}")
-    jobs = jobs or min(len(srcs), max(1, min(16, os.cpu_count() or 1)))
+    jobs = jobs or min(len(srcs) + 1, max(1, min(16, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        native = pool.submit(_compile_native, verbose)
         objs = list(pool.map(lambda s: _compile(s, verbose), srcs))
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
@@ -98,6 +140,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, LIB_PATH)
+    _link_native(native.result(), verbose)
     return LIB_PATH
 
 

@@ -113,6 +113,17 @@ def _use_hip_append(backend: str, cache: torch.Tensor) -> bool:
             and _hip.is_gfx950(cache.device) and _hip.library_available())
 
 
+def _fuses_plainly(cache, q, new_k, new_v, append_backend: str, attention_backend: str) -> bool:
+    """Whether ``append_and_attend`` of these tensors passes every check but
+    the lengths and takes the fused append + decode: the usual step, checked
+    natively (a fifth of the host time of the checks written out below)."""
+    return (append_backend in ("auto", "fused") and attention_backend in ("auto", "hip", "triton")
+            and not torch.compiler.is_compiling()
+            and _hip.native().step_args(q, cache.k, cache.v, new_k, new_v) is True
+            and (append_backend == "fused"
+                 or os.environ.get("KOTFLASH_ENABLE_CUDA_APPEND") != "0"))
+
+
 class PreallocatedKVCache:
     """Fixed-capacity K/V storage with append-only writes (reference
     kotflash/cache.py:91-290).
@@ -203,6 +214,16 @@ class PreallocatedKVCache:
         autograd. ``"auto"`` takes it whenever it applies (``_auto_fuses``),
         else appends with the HIP kernel or torch copies and attends.
         """
+        if (_fuses_plainly(self, q_new, new_k, new_v, append_backend, attention_backend)
+                and q_new.shape[2] == 1 and new_k.shape[2] == 1 and self.length < self.max_len):
+            from .kernels import hip_decode
+
+            output = hip_decode.attention_forward_strided_append(
+                q_new, self.k, self.v, new_k, new_v,
+                past_length=self.length, scale=1.0 / (self.k.shape[-1] ** 0.5),
+            )
+            self.length += 1
+            return output
         if attention_backend not in ("auto", "hip", "triton", "sdpa"):
             raise ValueError("attention backend must be one of: auto, hip, triton or sdpa")
         if append_backend not in ("auto", "torch", "hip", "cuda", "fused"):
@@ -272,14 +293,44 @@ class RaggedKVCache(PreallocatedKVCache):
             raise ValueError(f"lengths must be in [0, max_len={self.max_len}]")
         self._set(lengths)
 
-    def _set(self, lengths: List[int]) -> None:
+    # Stream (raw handle) of the last append, whose tokens and lengths a call
+    # on another stream has to wait for; None when the host has waited.
+    _writer = None
+
+    def _order_streams(self) -> None:
+        """Make the current stream wait for the last append if that ran on
+        another one. (Under graph capture nothing may be waited for; starting
+        a capture synchronizes with the device.)"""
+        if self._writer is None or _hip._stream(self.k.device) == self._writer \
+                or torch.cuda.is_current_stream_capturing():
+            return
+        dev = self.k.device
+        other = (torch.cuda.default_stream(dev) if self._writer == 0
+                 else torch.cuda.ExternalStream(self._writer, device=dev))
+        torch.cuda.current_stream(dev).wait_stream(other)
+
+    def _set(self, lengths: List[int], wait: bool = True) -> None:
+        """Set the lengths on the host and in the device mirrors. ``wait``:
+        return once the mirrors are written, whatever stream reads them next;
+        an append (``wait=False``) only orders them after its own writes, on
+        its stream."""
         self.lengths = lengths
         self.length = max(lengths) if lengths else 0
+        if not torch.compiler.is_compiling() \
+                and _hip.native().store_lengths(self.starts, self.seqlens, lengths) is None:
+            if wait:
+                torch.cuda.current_stream(self.k.device).synchronize()
+                self._writer = None
+            else:
+                self._writer = _hip._stream(self.k.device)
+            return
+        self._writer = None
         host = torch.tensor(lengths, dtype=torch.int64)
         self.starts.copy_(host, non_blocking=False)
         self.seqlens.copy_(host.to(torch.int32), non_blocking=False)
 
     def append(self, new_k: torch.Tensor, new_v: torch.Tensor, *, backend: str = "auto") -> None:
+        self._order_streams()
         self._check_new(new_k, new_v)
         if backend not in APPEND_BACKENDS:
             raise ValueError("append backend must be one of: auto, torch, hip or cuda")
@@ -299,7 +350,7 @@ class RaggedKVCache(PreallocatedKVCache):
             for b, start in enumerate(self.lengths):
                 self.k[b, :, start:start + n].copy_(new_k[b])
                 self.v[b, :, start:start + n].copy_(new_v[b])
-        self._set([x + n for x in self.lengths])
+        self._set([x + n for x in self.lengths], wait=False)
 
     def append_and_attend(self, q_new, new_k, new_v, *, append_backend: str = "auto",
                           attention_backend: str = "auto") -> torch.Tensor:
@@ -313,6 +364,18 @@ class RaggedKVCache(PreallocatedKVCache):
         otherwise it appends (``append``) and attends (``attend``) as two
         steps.
         """
+        self._order_streams()
+        if (_fuses_plainly(self, q_new, new_k, new_v, append_backend, attention_backend)
+                and max(self.lengths) + new_k.shape[2] <= self.max_len):
+            from .kernels import hip_decode
+
+            n = new_k.shape[2]
+            out = hip_decode.attention_append_decode_ragged(
+                q_new, self.k, self.v, new_k, new_v, self.seqlens, host_lengths=self.lengths,
+                scale=1.0 / (q_new.shape[-1] ** 0.5),
+            )
+            self._set([x + n for x in self.lengths], wait=False)
+            return out
         if attention_backend not in ("auto", "hip", "triton", "sdpa"):
             raise ValueError("attention backend must be one of: auto, hip, triton or sdpa")
         if append_backend not in ("auto", "torch", "hip", "cuda", "fused"):
@@ -350,7 +413,7 @@ class RaggedKVCache(PreallocatedKVCache):
                 q_new, self.k, self.v, new_k, new_v, self.seqlens, host_lengths=self.lengths,
                 scale=1.0 / (q_new.shape[-1] ** 0.5),
             )
-            self._set([x + n for x in self.lengths])
+            self._set([x + n for x in self.lengths], wait=False)
             return out
         self.append(new_k, new_v, backend=append_backend)
         return self.attend(q_new, backend=attention_backend)
@@ -366,6 +429,7 @@ class RaggedKVCache(PreallocatedKVCache):
         """Non-causal decode of q [B, Hq, Sq, D]; rows of sequence b see its
         first lengths[b] positions. HIP: one split-KV decode launch for all
         sequences; SDPA: one call per sequence."""
+        self._order_streams()
         if not isinstance(q, torch.Tensor) or q.ndim != 4:
             raise ValueError("q must use [B, Hq, Sq, D] layout")
         if q.shape[0] != self.k.shape[0] or q.shape[-1] != self.k.shape[-1]:

@@ -62,9 +62,43 @@ __global__ __launch_bounds__(256) void append_kernel(const AppendParams p) {
   }
 }
 
+// Per-sequence lengths of a ragged cache, from the host by value (kernel
+// arguments): one launch and no copy to wait for. Launch-bound.
+constexpr int kLenBatch = 256;
+struct Lengths {
+  int32_t v[kLenBatch];
+};
+__global__ __launch_bounds__(kLenBatch) void store_lengths_kernel(int64_t* starts, int32_t* seqlens, int n,
+                                                                  const Lengths len) {
+  const int i = threadIdx.x;
+  if (i >= n) return;
+  starts[i] = len.v[i];
+  seqlens[i] = len.v[i];
+}
+
 }  // namespace kf
 
 using namespace kf;
+
+extern "C" int kf_store_lengths(int64_t* starts, int32_t* seqlens, const int32_t* lengths, int64_t count,
+                                void* stream) {
+  const char* what = "kf_store_lengths";
+  if (starts == nullptr || seqlens == nullptr || lengths == nullptr)
+    return set_error(KF_EINVAL, "%s: null pointer", what);
+  if (count <= 0) return set_error(KF_EINVAL, "%s: count must be positive", what);
+  for (int64_t i = 0; i < count; ++i)
+    if (lengths[i] < 0) return set_error(KF_EINVAL, "%s: lengths must be non-negative", what);
+  for (int64_t i = 0; i < count; i += kLenBatch) {
+    const int n = (int)(count - i < kLenBatch ? count - i : kLenBatch);
+    Lengths len{};
+    for (int j = 0; j < n; ++j) len.v[j] = lengths[i + j];
+    hipLaunchKernelGGL(store_lengths_kernel, dim3(1), dim3(kLenBatch), 0, (hipStream_t)stream, starts + i,
+                       seqlens + i, n, len);
+    const int rc = check_launch(what);
+    if (rc) return rc;
+  }
+  return KF_OK;
+}
 
 extern "C" int kf_kv_append(void* k_cache, void* v_cache, const void* new_k, const void* new_v,
                             const int64_t* start_dev, int64_t start, int64_t B, int64_t H,

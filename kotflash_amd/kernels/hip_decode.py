@@ -114,6 +114,10 @@ def attention_forward_strided_append(q, k_cache, v_cache, new_k, new_v, *,
     other splits read positions [0, past_length) in place. Head dims that are
     not a multiple of 8 take a separate append launch and a padded decode.
     """
+    if not torch.compiler.is_compiling():
+        out = _hip.native().append_step(q, k_cache, v_cache, new_k, new_v, past_length, scale)
+        if out is not NotImplemented:
+            return out
     require_hip_tensors("fused append/decode", q, k_cache, v_cache, new_k, new_v)
     if q.ndim != 4 or q.shape[2] != 1:
         raise ValueError("q must be [B,Hq,1,D]")
@@ -180,6 +184,11 @@ def attention_append_decode_ragged(q, k_cache, v_cache, new_k, new_v, seqlens: t
     seqlens[b] + n positions after the append: one decode launch and one
     merge (``kf_attn_append_decode``). Callers validate capacity first.
     Returns O, or (O, LSE) with ``with_lse``."""
+    if not with_lse and not torch.compiler.is_compiling():
+        out = _hip.native().append_ragged(q, k_cache, v_cache, new_k, new_v, seqlens, host_lengths,
+                                          scale)
+        if out is not NotImplemented:
+            return out
     require_hip_tensors("ragged append/decode", q, k_cache, v_cache, new_k, new_v)
     if seqlens.dtype != torch.int32 or seqlens.device != q.device or seqlens.shape != (q.shape[0],):
         raise ValueError("seqlens must be a device int32 tensor of shape [B]")
@@ -218,6 +227,11 @@ def attention_decode_ragged(q, k_cache, v_cache, seqlens: torch.Tensor, *, max_s
     (the same lengths on the host, with max == max_seqlen) lets the planner
     size the splits from the total visible work. Returns O, or (O, LSE) with
     ``with_lse``."""
+    if (not with_lse and isinstance(host_lengths, list) and host_lengths
+            and not torch.compiler.is_compiling() and max(host_lengths) == max_seqlen):
+        out = _hip.native().decode_ragged(q, k_cache, v_cache, seqlens, host_lengths, scale)
+        if out is not NotImplemented:
+            return out
     require_hip_tensors("ragged decode", q, k_cache, v_cache)
     if seqlens.dtype != torch.int32 or seqlens.device != q.device or seqlens.shape != (q.shape[0],):
         raise ValueError("seqlens must be a device int32 tensor of shape [B]")
