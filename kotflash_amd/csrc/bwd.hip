@@ -11,7 +11,7 @@
 //      SIMD): per key tile it recomputes S^T = K Q^T and dP^T = V dO^T, forms
 //      dS^T = P^T (dP^T - delta) with P = exp(scale S - LSE), and accumulates
 //      dQ^T += K^T dS^T; dQ = scale * dQ (reference :17-91). Short problems
-//      take a split form: 32 rows per workgroup, the waves splitting the key
+//      take split forms (RB x KG, attn_form): key groups splitting the key
 //      range, their dQ summed through LDS.
 //   3. dkdv_kernel (key-stationary, 4 waves, one per SIMD): a key tile is 128
 //      keys of one (batch, kv_head); wave w keeps keys 32 w .. +31 in
@@ -70,6 +70,7 @@ struct BwdParams {
   int G, ngroups;
   int nqt, nkt;    // dq: 128-row query tiles; dkdv: 64-row query tiles, 128-key tiles
   int nwg;         // dkdv workgroups (stream-K share count)
+  int fold;        // dq: the whole grid is resident at once (fold_rank)
   int64_t units;   // dkdv: total (KV group, key tile, head, query tile) units
   float scale, scale_log2;
 };
@@ -188,6 +189,12 @@ __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
+// Waves per SIMD the dQ kernel is compiled for, and workgroups per CU.
+constexpr int dq_waves_per_simd(int DT, int RB, int KG) {
+  return RB * KG == 8 ? 2 : RB == 2 && DT <= 64 ? 2 : KG > 1 ? 1 : 2;
+}
+constexpr int dq_wgs_per_cu(int DT, int RB, int KG) { return dq_waves_per_simd(DT, RB, KG) * 4 / (RB * KG); }
+
 // 2. dQ, query-stationary: 4 waves x 32 rows, 64-key tiles, two workgroups
 // per CU. Each 32-key block is finished (S, dP, dS, dQ update) before the next
 // starts so the live registers fit two waves per SIMD. K/V tiles stream into
@@ -198,15 +205,21 @@ __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
 // deltas): DT / 16, or 5 for head dims up to 80 in a 96-wide tile, whose
 // last 16 columns are zero padding.
 //
-// SPLIT (short problems, the forward's split form): the workgroup owns 32
-// query rows and its four waves split the key range, wave w taking tiles w,
-// w + 4, ... through a ring of its own (two stages up to head dim 64, one
-// above, where the next tile's V loads after the S/dP product and its K after
-// the dQ product). The four fp32 dQ are summed through LDS; P already uses
-// the global LSE, so no weights are needed. Wave 0 writes the row deltas.
-template <typename T, int DT, int KS, bool CAUSAL, bool SPLIT>
-__global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams p) {
-  constexpr int BM = SPLIT ? 32 : 128;
+// RB x KG: row blocks and key groups of a workgroup, as in the forward (4x1
+// is the tiled form). Wave (rb, kg) takes tiles kg, kg + KG, ... through its
+// group's ring (two stages, or one where two of every group exceed 128 KB,
+// where the next tile's V loads after the S/dP product and its K after the dQ
+// product). The groups' fp32 dQ are summed through LDS; P already uses the
+// global LSE, so no weights are needed. Group 0 writes the row deltas.
+// Measured against 4x1, us: B=1 Hq=16 S=2048 D=64 causal 29.5 -> 21.3 (2x2),
+// B=2 Hq=16 Sq=448 Sk=1500 D=64 22.6 -> 15.5 (2x4), B=1 Hq=16 S=1024 D=128
+// 36.2 -> 21.4 (2x2, 27.7 of the 4x1 with its reloads removed).
+template <typename T, int DT, int KS, bool CAUSAL, int RB, int KG>
+__global__ __launch_bounds__(64 * RB * KG, dq_waves_per_simd(DT, RB, KG)) void dq_kernel(const BwdParams p) {
+  constexpr bool SPLIT = KG > 1;
+  constexpr bool SHARED = RB > 1;       // a group's ring is shared by RB waves
+  constexpr int NW = RB * KG;           // waves per workgroup
+  constexpr int BM = 32 * RB;
   constexpr int BN = 64;
   constexpr int CPR = DT / 8;
   constexpr int NKS = KS;
@@ -219,35 +232,41 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
   constexpr int NDB = TAIL ? 2 : DT / 32;
   constexpr int TB = BN * DT * 2;       // bytes of one K (or V) tile
   constexpr int STAGE_B = 2 * TB;       // K | V
-  constexpr int NST = (SPLIT && DT > 64) ? 1 : 2;  // ring stages
-  // 1 KB loads per wave per tile and matrix: a quarter of the tile, or all of
-  // it in the split form.
-  constexpr int NKI = BN * CPR / (SPLIT ? 64 : 256);
-  static_assert(BN * CPR == (SPLIT ? 64 : 256) * NKI, "tile chunks must split into whole loads");
-  constexpr int RING_B = (SPLIT ? 4 : 1) * NST * STAGE_B;
-  constexpr int OSTR = DT + 1;  // split form: per-wave dQ^T rows in LDS
-  constexpr int MERGE_B = SPLIT ? 4 * 32 * OSTR * 4 : 0;
+  constexpr int NST = KG * 2 * STAGE_B <= 128 * 1024 ? 2 : 1;  // ring stages
+  static_assert(NST == 2 || !SHARED, "a one-stage ring belongs to one wave");
+  // 1 KB loads per wave per tile and matrix: the tile over the group's waves.
+  constexpr int NKI = BN * CPR / (64 * RB);
+  static_assert(BN * CPR == 64 * RB * NKI, "tile chunks must split into whole loads");
+  constexpr int RING_B = KG * NST * STAGE_B;
+  constexpr int OSTR = DT + 1;  // KG > 1: per-wave dQ^T rows in LDS
+  constexpr int MERGE_B = SPLIT ? NW * 32 * OSTR * 4 : 0;
   constexpr int SMEM_B = RING_B > MERGE_B ? RING_B : MERGE_B;
   using Tile = SwizzledTile<CPR>;
   __shared__ __attribute__((aligned(16))) uint16_t smem[SMEM_B / 2];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
+  const int rb = RB == 1 ? 0 : KG == 1 ? wave : wave % RB;  // row block
+  const int kg = KG == 1 ? 0 : RB == 1 ? wave : wave / RB;  // key group
   const int l32 = lane & 31, h32 = lane >> 5;
 
   // Longest query tiles first; KV groups kept on one XCD as in the forward.
   int qt, b, h;
   {
-    const int bid = blockIdx.x;
+    int bid = blockIdx.x;
+    const int fold = CAUSAL ? p.fold : 0;
     if ((p.ngroups & 7) == 0) {
-      const int x = bid & 7, j = bid >> 3, gpx = p.ngroups >> 3, per_tile = p.G * gpx;
+      const int x = bid & 7, gpx = p.ngroups >> 3, per_tile = p.G * gpx;
+      const int j = fold_rank<32>(bid >> 3, per_tile * p.nqt, fold);
       const int t = j / per_tile, r = j - t * per_tile;
       qt = p.nqt - 1 - t;
       const int grp = x + 8 * (r / p.G);
       b = grp / p.Hkv;
       h = (grp % p.Hkv) * p.G + r % p.G;
     } else {
-      const int bh = p.B * p.Hq, t = bid / bh, r = bid - t * bh;
+      const int bh = p.B * p.Hq;
+      bid = fold_rank<256>(bid, bh * p.nqt, fold);
+      const int t = bid / bh, r = bid - t * bh;
       qt = p.nqt - 1 - t;
       b = r / p.Hq;
       h = r % p.Hq;
@@ -255,7 +274,7 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
   }
   const int kvh = h / p.G;
   const int q0 = qt * BM;
-  const int qrow = q0 + (SPLIT ? 0 : wave * 32) + l32;
+  const int qrow = q0 + rb * 32 + l32;
   const bool row_ok = qrow < p.Sq;
 
   const auto qr = make_rsrc(p.q + b * p.q_sb + h * p.q_sh, rows_extent(p.Sq, p.q_ss, p.D));
@@ -295,7 +314,7 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
         dlt += Elem<T>::to_f32((uint16_t)(of[ks][w] >> 16)) * Elem<T>::to_f32((uint16_t)(dof[ks][w] >> 16));
       }
     dlt = wave_xor32_sum(dlt);
-    if (row_ok && h32 == 0 && (!SPLIT || wave == 0)) {
+    if (row_ok && h32 == 0 && kg == 0) {
       p.delta[rowlin] = -dlt;
       p.lse2[rowlin] = lse2;
     }
@@ -310,9 +329,11 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
 
   const int nkeys = CAUSAL ? min(p.Sk, q0 + BM) : p.Sk;
   const int ntiles = cdiv(nkeys, BN);
-  // This wave's tiles: all of them, or every fourth from tile `wave`.
-  const int nl = SPLIT ? (ntiles > wave ? (ntiles - wave + 3) / 4 : 0) : ntiles;
-  auto tile_of = [&](int li) { return SPLIT ? wave + 4 * li : li; };
+  // This group's tiles: kg, kg + KG, ... Waves that share rings step together
+  // (nloop bodies, the same for every group).
+  const int nl = KG == 1 ? ntiles : ntiles > kg ? (ntiles - kg + KG - 1) / KG : 0;
+  const int nloop = KG > 1 && SHARED ? cdiv(ntiles, KG) : nl;
+  auto tile_of = [&](int li) { return kg + KG * li; };
 
   // Per-lane load plan: for each of this wave's NKI 1 KB blocks of a tile,
   // the byte offset of this lane's 16-byte chunk within the tile's rows
@@ -321,18 +342,18 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
   uint32_t koff[NKI], voff[NKI];
 #pragma unroll
   for (int k = 0; k < NKI; ++k) {
-    const int pc = ((SPLIT ? 0 : wave * NKI) + k) * 64 + lane;
+    const int pc = (rb * NKI + k) * 64 + lane;
     const int r = pc / CPR;
     const int c = (pc % CPR) ^ Tile::key(r);
     const bool ok = c * 8 < p.D;
     koff[k] = ok ? (uint32_t)(r * p.k_ss + c * 8) * 2u : kOOB;
     voff[k] = ok ? (uint32_t)(r * p.v_ss + c * 8) * 2u : kOOB;
   }
-  const uint32_t lds0 = lds_addr(smem) + (SPLIT ? (uint32_t)(wave * NST * STAGE_B) : 0u);
+  const uint32_t lds0 = lds_addr(smem) + (uint32_t)(kg * NST * STAGE_B);
   auto tile_load = [&](int tile, int st) {
     const uint32_t kso = (uint32_t)(tile * BN * p.k_ss) * 2u;
     const uint32_t vso = (uint32_t)(tile * BN * p.v_ss) * 2u;
-    const uint32_t m0 = lds0 + (uint32_t)st * STAGE_B + (SPLIT ? 0u : (uint32_t)(wave * NKI) * 1024u);
+    const uint32_t m0 = lds0 + (uint32_t)st * STAGE_B + (uint32_t)(rb * NKI) * 1024u;
 #pragma unroll
     for (int k = 0; k < NKI; ++k) {
       dma16_s(kr, m0 + k * 1024u, koff[k], kso);
@@ -381,23 +402,32 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
 
   if (nl > 0) tile_load(tile_of(0), 0);
   wait_all_memory();
-  if constexpr (!SPLIT) __syncthreads();
+  if constexpr (SHARED) __syncthreads();
 
-  const int wq0 = q0 + (SPLIT ? 0 : wave * 32);
+  const int wq0 = q0 + rb * 32;
   // This wave's li-th tile on ring stage ST (a compile-time constant, so
   // every LDS offset below is an immediate).
+  // Where a tile's body issues the next tile's loads: first, or (LATE) after
+  // its own first operand reads. A tile whose first key block lies above all
+  // of a wave's rows is its group's last, so a late wave misses no load.
+  // Measured, tiled form: after the reads the 64-wide tile runs 1.2-1.9%
+  // faster causal (B=2 Hq=16 Hkv=4 S=4096) and level non-causal, and the
+  // causal 128-wide one 4.3% in bf16 (174.5 against 181.9 us there) but 2%
+  // slower in fp16; the others are level or up to 1% slower.
+  constexpr bool LATE = KG == 1 && CAUSAL && (DT == 64 || (DT == 128 && std::is_same_v<T, __bf16>));
   auto tile_body = [&](int li, auto stc) {
     constexpr int ST = decltype(stc)::value;
     if constexpr (NST == 2) {
-      if (li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
+      if (!LATE && li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
     }
     const int kbase = tile_of(li) * BN;
     const bool need_mask = (kbase + BN > p.Sk) || (CAUSAL && kbase + BN - 1 > wq0);
+    const bool mine = !SHARED || KG == 1 || li < nl;  // false past the group's last tile
     bool v_next = false;  // one-stage ring: the next tile's V already issued
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       const int kb0 = kbase + 32 * kb;
-      if (CAUSAL && kb0 > wq0 + 31) continue;  // block entirely above the wave's rows
+      if (!mine || (CAUSAL && kb0 > wq0 + 31)) continue;  // block entirely above the wave's rows
       // S^T and dP^T as one stream of 2 NKS MFMA slots (slot m: k-step m / 2,
       // S for even m, dP for odd), then dQ^T as NDQ slots (head-dim block
       // j / 2, key half j % 2). Each slot issues the LDS read of the operand
@@ -415,7 +445,7 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
       // one reload inside the tile loop restores a DMA offset right after the
       // tile-end vmcnt(0) and barrier, so it drains nothing that was not
       // drained already. Narrower tiles stay at 4.
-      constexpr int LA = DT == 128 ? 5 : 4;
+      constexpr int LA = DT == 128 && NW == 4 ? 5 : 4;
       u32x4 op[NSD + NDQ];
       auto read_op = [&](int m) {
         if (m < NSD) {
@@ -444,11 +474,14 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
       // loads drained the ring eight times a tile (dQ at B=4 H=12 S=2048 D=128
       // non-causal: bf16 183.4 -> 137.6 us, fp16 188.8 -> 145.9). The other
       // kernels have no such spill and are faster keeping the copies.
-      if constexpr (!CAUSAL && DT == 128 && !SPLIT) asm volatile("" : "+v"(nd));
+      if constexpr (!CAUSAL && DT == 128 && RB == 4) asm volatile("" : "+v"(nd));
 #pragma unroll
       for (int r = 0; r < 16; ++r) dp[r] = nd;
       static_for<0, LA>([&](auto mc) { read_op(decltype(mc)::value); });
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (LATE) {
+        if (kb == 0 && li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
+      }
       // Raised priority while this wave issues MFMAs, so that the other wave
       // on the SIMD runs its softmax in the gaps instead of competing for them.
       __builtin_amdgcn_s_setprio(1);
@@ -539,15 +572,15 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
     KF_WAIT_VMCNT(0);  // this wave's loads of the next tile
     // Every wave's loads landed; stage ST is free again. The split form's
     // rings are per wave, and the wave's own wait suffices.
-    if constexpr (!SPLIT) __syncthreads();
+    if constexpr (SHARED) __syncthreads();
   };
   if constexpr (NST == 2) {
-    for (int li = 0; li < nl; li += 2) {
+    for (int li = 0; li < nloop; li += 2) {
       tile_body(li, std::integral_constant<int, 0>{});
-      if (li + 1 < nl) tile_body(li + 1, std::integral_constant<int, 1>{});
+      if (li + 1 < nloop) tile_body(li + 1, std::integral_constant<int, 1>{});
     }
   } else {
-    for (int li = 0; li < nl; ++li) tile_body(li, std::integral_constant<int, 0>{});
+    for (int li = 0; li < nloop; ++li) tile_body(li, std::integral_constant<int, 0>{});
   }
 
   if constexpr (SPLIT) {
@@ -563,21 +596,22 @@ __global__ __launch_bounds__(256, SPLIT ? 1 : 2) void dq_kernel(const BwdParams 
         for (int r = 0; r < 16; ++r) orow[32 * db + 8 * (r >> 2) + 4 * h32 + (r & 3)] = dq[db][r];
     }
     __syncthreads();
-    // Wave w stores head-dim columns [w DT/4, (w + 1) DT/4) of the 32 rows;
-    // a lane takes row l32 and half h32 of those columns.
-    constexpr int CW = DT / 4, CH = CW / 2;
+    // The KG waves of row block rb (waves rb + RB g) store its head-dim
+    // columns [kg DT/KG, (kg + 1) DT/KG); a lane takes row l32 and half h32 of
+    // those columns.
+    constexpr int CW = DT / KG, CH = CW / 2;
     static_assert(CH % 4 == 0, "stores are 4 columns wide");
     if (row_ok) {
       uint16_t* Dq = p.dq + b * p.dq_sb + h * p.dq_sh + qrow * p.dq_ss;
-      const int c0 = wave * CW + h32 * CH;
+      const int c0 = kg * CW + h32 * CH;
 #pragma unroll
       for (int j = 0; j < CH; j += 4) {
         const int d = c0 + j;
         if (d < p.D) {
           float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const float* src = ob + (w * 32 + l32) * OSTR + d;
+          for (int g = 0; g < KG; ++g) {
+            const float* src = ob + ((rb + RB * g) * 32 + l32) * OSTR + d;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] += src[e];
           }
@@ -1373,6 +1407,18 @@ static size_t partial_bytes(int nwg, int64_t D) {
   return (size_t)2 * nwg * 2 * kBNK * head_tile(D) * sizeof(float);
 }
 
+template <typename T, int DT, int KS, int RB, int KG>
+static int launch_dq_form(BwdParams p, bool causal, hipStream_t stream) {
+  p.nqt = cdiv(p.Sq, 32 * RB);
+  const dim3 grid((unsigned)((int64_t)p.nqt * p.B * p.Hq)), blk(64 * RB * KG);
+  p.fold = fold_tiles(p.nqt, grid.x, dq_wgs_per_cu(DT, RB, KG));
+  if (causal)
+    hipLaunchKernelGGL((dq_kernel<T, DT, KS, true, RB, KG>), grid, blk, 0, stream, p);
+  else
+    hipLaunchKernelGGL((dq_kernel<T, DT, KS, false, RB, KG>), grid, blk, 0, stream, p);
+  return check_launch("kf_attn_bwd(dq)");
+}
+
 template <typename T, int DT, int KS>
 static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) {
   // dq_kernel computes the row deltas itself: the delta launch is only needed
@@ -1384,23 +1430,19 @@ static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) 
     if (rc) return rc;
   }
   if (stages & KF_BWD_DQ) {
-    // The forward's rule for its split form: grids of 128-row tiles that
-    // leave most CUs idle take 32-row workgroups whose waves split the key
-    // range.
-    const bool split = attn_use_split(p.B, p.Hq, p.Sq, p.Sk, causal);
-    p.nqt = cdiv(p.Sq, split ? 32 : 128);
-    const int64_t gq = (int64_t)p.nqt * p.B * p.Hq;
-    if (split) {
-      if (causal)
-        hipLaunchKernelGGL((dq_kernel<T, DT, KS, true, true>), dim3((unsigned)gq), dim3(256), 0, stream, p);
-      else
-        hipLaunchKernelGGL((dq_kernel<T, DT, KS, false, true>), dim3((unsigned)gq), dim3(256), 0, stream, p);
-    } else if (causal) {
-      hipLaunchKernelGGL((dq_kernel<T, DT, KS, true, false>), dim3((unsigned)gq), dim3(256), 0, stream, p);
-    } else {
-      hipLaunchKernelGGL((dq_kernel<T, DT, KS, false, false>), dim3((unsigned)gq), dim3(256), 0, stream, p);
+    int rc = KF_OK;
+    switch (attn_form(kDqCosts[DT / 32 - 1], p.B * p.Hq, p.Sq, p.Sk, causal)) {
+      case kForm4x2: rc = launch_dq_form<T, DT, KS, 4, 2>(p, causal, stream); break;
+      case kForm2x2: rc = launch_dq_form<T, DT, KS, 2, 2>(p, causal, stream); break;
+      case kForm2x4:
+        if constexpr (DT <= 64) rc = launch_dq_form<T, DT, KS, 2, 4>(p, causal, stream);
+        break;
+      case kForm1x8:
+        if constexpr (DT == 64) rc = launch_dq_form<T, DT, KS, 1, 8>(p, causal, stream);
+        break;
+      case kForm1x4: rc = launch_dq_form<T, DT, KS, 1, 4>(p, causal, stream); break;
+      default: rc = launch_dq_form<T, DT, KS, 4, 1>(p, causal, stream); break;
     }
-    int rc = check_launch("kf_attn_bwd(dq)");
     if (rc) return rc;
   }
   if (stages & KF_BWD_DKDV) {

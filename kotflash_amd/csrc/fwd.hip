@@ -1,15 +1,15 @@
 // Attention forward for gfx950: online softmax with MFMA QK^T and PV.
 //
-// Work decomposition. One workgroup (4 waves) owns BM = 4 * QB * 32 query rows
-// of one (batch, q_head). Each wave owns QB blocks of 32 rows and keeps them
-// for the whole kernel:
+// Work decomposition. A workgroup owns RB blocks of 32 query rows of one
+// (batch, q_head), each block by KG waves that split its keys (RB x KG is the
+// kernel's form, chosen by attn_form; 4x1 for large problems). Each wave keeps
+// its 32 rows for the whole kernel:
 //   - Q rows in registers as MFMA B operands,
 //   - the running max m, the running denominator l and the output accumulator
 //     O^T (head_dim x rows) in registers.
 // The workgroup streams K/V in tiles of BN = 64 keys through a two-stage LDS
 // ring filled by direct-to-LDS loads one tile ahead, so one barrier per tile
-// suffices. Short problems take the split form (SPLIT, below): 32 rows per
-// workgroup, the four waves splitting the key range.
+// suffices. With KG > 1 every key group has a ring of its own.
 //
 // Per tile and 32-row block the wave computes S^T = K Q^T (keys x rows), so a
 // lane owns one query row and 32 of the tile's 64 scores in registers: the row
@@ -44,6 +44,7 @@ struct FwdParams {
   int64_t o_sb, o_sh, o_ss;
   int B, Hq, Hkv, Sq, Sk, D;
   int nqt;
+  int fold;  // 1: the whole grid is resident at once (fold_rank)
   float scale_log2;
 };
 
@@ -52,14 +53,15 @@ struct FwdParams {
 // groups is a multiple of the 8 XCDs, the workgroups of one KV group are kept
 // on one XCD (the dispatcher assigns block i to XCD i % 8) so its L2 serves the
 // group's K/V to all of them.
-__device__ inline void fwd_map_block(int bid, int nqt, int B, int Hq, int Hkv, int& qt, int& b,
+__device__ inline void fwd_map_block(int bid, int nqt, int B, int Hq, int Hkv, int fold, int& qt, int& b,
                                      int& h) {
   const int G = Hq / Hkv;
   const int ngroups = B * Hkv;
   if ((ngroups & 7) == 0) {
-    const int x = bid & 7, j = bid >> 3;
     const int gpx = ngroups >> 3;
     const int per_tile = G * gpx;
+    const int x = bid & 7;
+    const int j = fold_rank<32>(bid >> 3, per_tile * nqt, fold);
     const int t = j / per_tile, r = j - t * per_tile;
     qt = nqt - 1 - t;
     const int grp = x + 8 * (r / G);
@@ -68,6 +70,7 @@ __device__ inline void fwd_map_block(int bid, int nqt, int B, int Hq, int Hkv, i
     h = (grp % Hkv) * G + g;
   } else {
     const int bh = B * Hq;
+    bid = fold_rank<256>(bid, bh * nqt, fold);
     const int t = bid / bh, r = bid - t * bh;
     qt = nqt - 1 - t;
     b = r / Hq;
@@ -75,29 +78,43 @@ __device__ inline void fwd_map_block(int bid, int nqt, int B, int Hq, int Hkv, i
   }
 }
 
+// Waves per SIMD the kernel is compiled for.
+constexpr int fwd_waves_per_simd(int DT, int RB, int KG) {
+  return RB * KG == 8 ? 2 : RB == 2 && DT <= 64 ? 2 : KG > 1 ? 1 : DT == 96 ? 3 : 2;
+}
+
 // KS is the number of 16-column k-steps of the S = K Q^T contraction: DT / 16,
 // or fewer when the head dim ends earlier inside the tile (D <= 80 in a
 // 96-wide tile needs 5): the skipped columns are zero padding on both sides.
 //
-// SPLIT (short problems, where 128-row tiles leave most CUs idle): the
-// workgroup owns 32 query rows and its four waves split the key range
-// instead, wave w taking K/V tiles w, w + 4, ... through a ring of its own in
-// LDS (no workgroup barrier per tile). Each wave ends with its own (m, l, O)
-// over its tiles; they are combined through LDS with the LSE weights
-// 2^(m_w - M) / sum_w l_w 2^(m_w - M), as split-KV partials are (reference
-// triton_forward.py:269-349). The longest chain of dependent tiles is a
-// quarter of the unsplit kernel's, and the grid four times as large.
+// KG > 1 (short problems, where 128-row tiles leave CUs idle): wave (rb, kg)
+// owns row block rb and takes K/V tiles kg, kg + KG, ... through its group's
+// ring in LDS, which it shares with the group's other row blocks (RB = 1: its
+// own, without a workgroup barrier per tile). Each wave ends with its own
+// (m, l, O) over its tiles; the groups' are combined through LDS with the LSE
+// weights 2^(m_g - M) / sum_g l_g 2^(m_g - M), as split-KV partials are
+// (reference triton_forward.py:269-349). The longest chain of dependent tiles
+// is KG times shorter. What bounds these forms: a wave alone on its SIMD takes
+// 0.7 us (D = 64) to 1.1 us (D = 128) per tile, most of it latency; with fewer
+// row blocks per ring more K/V bytes cross from L2 (about 45 B per clock and
+// CU is the most that arrived). Measured against 4x1 or 1x4, us: B=1 Hq=16
+// S=2048 D=64 causal 26.9 -> 18.0 (2x2), B=2 Hq=16 Sq=448 Sk=1500 D=64
+// 20.5 -> 12.8 (2x4), B=2 Hq=16 Sq=100 Sk=3000 D=64 14.0 -> 12.4 (1x8), B=1
+// Hq=16 S=2048 D=128 causal 39.2 -> 32.6 (4x2).
 //
-// Occupancy: two workgroups per CU, or three for the 96-wide tile (48 KB of
+// Occupancy of the tiled form (4x1): two workgroups per CU, or three for the 96-wide tile (48 KB of
 // LDS each, and 168 VGPRs with a 16-byte spill outside the tile loop). Three
 // took the config 4 forward (768 equal tiles, one and a half rounds at two
 // per CU) 3.5-5% faster at D = 72 and 96 and a causal D = 96 grid of 1024
 // tiles 3% faster, bit-identical; the 64- and 32-wide tiles fit three too
 // but ran within 0.2% of two, and the 128-wide tile's LDS does not fit.
-template <typename T, int DT, int KS, int QB, bool CAUSAL, bool SPLIT>
-__global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)) void fwd_kernel(const FwdParams p) {
-  static_assert(!SPLIT || QB == 1, "the split form has one 32-row block per workgroup");
-  constexpr int BM = SPLIT ? 32 : 4 * QB * 32;
+template <typename T, int DT, int KS, bool CAUSAL, int RB, int KG>
+__global__ __launch_bounds__(64 * RB * KG, fwd_waves_per_simd(DT, RB, KG)) void fwd_kernel(const FwdParams p) {
+  constexpr int QB = 1;                 // 32-row blocks per wave
+  constexpr bool SPLIT = KG > 1;
+  constexpr bool SHARED = RB > 1;       // a group's ring is shared by RB waves
+  constexpr int NW = RB * KG;           // waves per workgroup
+  constexpr int BM = 32 * RB;
   constexpr int BN = 64;
   constexpr int CPR = DT / 8;           // 16-byte chunks per row
   constexpr int NKS = KS;               // MFMA k-steps over head_dim
@@ -105,37 +122,39 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
   // Head dims up to 80 in the 96-wide tile (TAIL): O^T columns 0-63 in two
   // 32-wide blocks and 64-79 as a 16-wide tail of v_mfma_f32_16x16x32
   // products, so the PV product runs 80 columns instead of 96 (the S product
-  // already stops at 80 through KS). The tiled form only; the split form
-  // keeps three 32-wide blocks.
+  // already stops at 80 through KS). Only with one key group; the others keep
+  // three 32-wide blocks.
   constexpr bool TAIL = DT == 96 && KS == 5 && !SPLIT;
   constexpr int NDB = TAIL ? 2 : DT / 32;  // 32-wide head_dim blocks of O^T
   constexpr int TB = BN * DT * 2;       // bytes of one K (or V) tile
   constexpr int STAGE_B = 2 * TB;       // K | V
-  // Ring stages: two, shared by the workgroup; in the split form one ring per
-  // wave, of two stages where four of them fit the LDS (head dims up to 64).
-  constexpr int NST = (SPLIT && DT > 64) ? 1 : 2;
-  // 1 KB loads per wave per tile and matrix: a quarter of the tile, or all of
-  // it in the split form.
-  constexpr int NKI = BN * CPR / (SPLIT ? 64 : 256);
-  static_assert(BN * CPR == (SPLIT ? 64 : 256) * NKI, "tile chunks must split into whole loads");
-  constexpr int RING_B = (SPLIT ? 4 : 1) * NST * STAGE_B;
+  // Ring stages of a group: two, or one where two of every group's exceed
+  // 128 KB of LDS (which only the forms with one row block reach).
+  constexpr int NST = KG * 2 * STAGE_B <= 128 * 1024 ? 2 : 1;
+  static_assert(NST == 2 || !SHARED, "a one-stage ring belongs to one wave");
+  // 1 KB loads per wave per tile and matrix: the tile over the group's waves.
+  constexpr int NKI = BN * CPR / (64 * RB);
+  static_assert(BN * CPR == 64 * RB * NKI, "tile chunks must split into whole loads");
+  constexpr int RING_B = KG * NST * STAGE_B;
   // Split form: the merge buffer (per wave O^T rows padded to DT + 1 floats,
   // then m and l per row) overlays the rings after the last tile.
   constexpr int OSTR = DT + 1;
-  constexpr int MERGE_B = SPLIT ? (4 * 32 * OSTR + 2 * 4 * 32) * 4 : 0;
+  constexpr int MERGE_B = SPLIT ? (NW * 32 * OSTR + 2 * NW * 32) * 4 : 0;
   constexpr int SMEM_B = RING_B > MERGE_B ? RING_B : MERGE_B;
   using Tile = SwizzledTile<CPR>;
   __shared__ __attribute__((aligned(16))) uint16_t smem[SMEM_B / 2];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = wave_index();
+  const int rb = RB == 1 ? 0 : KG == 1 ? wave : wave % RB;  // row block
+  const int kg = KG == 1 ? 0 : RB == 1 ? wave : wave / RB;  // key group
   const int l32 = lane & 31, h32 = lane >> 5;
 
   int qt, b, h;
-  fwd_map_block(blockIdx.x, p.nqt, p.B, p.Hq, p.Hkv, qt, b, h);
+  fwd_map_block(blockIdx.x, p.nqt, p.B, p.Hq, p.Hkv, CAUSAL ? p.fold : 0, qt, b, h);
   const int kvh = h / (p.Hq / p.Hkv);
   const int q0 = qt * BM;
-  const int wq0 = SPLIT ? q0 : q0 + wave * QB * 32;
+  const int wq0 = q0 + rb * 32;
 
   const auto qr = make_rsrc(p.q + b * p.q_sb + h * p.q_sh, rows_extent(p.Sq, p.q_ss, p.D));
   const auto kr = make_rsrc(p.k + b * p.k_sb + kvh * p.k_sh, rows_extent(p.Sk, p.k_ss, p.D));
@@ -180,9 +199,11 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
 
   const int nkeys = CAUSAL ? min(p.Sk, q0 + BM) : p.Sk;
   const int ntiles = cdiv(nkeys, BN);
-  // This wave's tiles: all of them, or every fourth from tile `wave`.
-  const int nl = SPLIT ? (ntiles > wave ? (ntiles - wave + 3) / 4 : 0) : ntiles;
-  auto tile_of = [&](int li) { return SPLIT ? wave + 4 * li : li; };
+  // This group's tiles: kg, kg + KG, ... Waves that share rings step together
+  // (nloop bodies, the same for every group).
+  const int nl = KG == 1 ? ntiles : ntiles > kg ? (ntiles - kg + KG - 1) / KG : 0;
+  const int nloop = KG > 1 && SHARED ? cdiv(ntiles, KG) : nl;
+  auto tile_of = [&](int li) { return kg + KG * li; };
 
   // K/V tiles stream into a two-stage LDS ring by direct-to-LDS loads, stored
   // unpadded with the swizzle of SwizzledTile (conflict-free for both the
@@ -194,18 +215,18 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
   uint32_t koff[NKI], voff[NKI];
 #pragma unroll
   for (int k = 0; k < NKI; ++k) {
-    const int pc = ((SPLIT ? 0 : wave * NKI) + k) * 64 + lane;
+    const int pc = (rb * NKI + k) * 64 + lane;
     const int r = pc / CPR;
     const int c = (pc % CPR) ^ Tile::key(r);
     const bool ok = c * 8 < p.D;
     koff[k] = ok ? (uint32_t)(r * p.k_ss + c * 8) * 2u : kOOB;
     voff[k] = ok ? (uint32_t)(r * p.v_ss + c * 8) * 2u : kOOB;
   }
-  const uint32_t lds0 = lds_addr(smem) + (SPLIT ? (uint32_t)(wave * NST * STAGE_B) : 0u);
+  const uint32_t lds0 = lds_addr(smem) + (uint32_t)(kg * NST * STAGE_B);
   auto tile_load = [&](int tile, int st) {
     const uint32_t kso = (uint32_t)(tile * BN * p.k_ss) * 2u;
     const uint32_t vso = (uint32_t)(tile * BN * p.v_ss) * 2u;
-    const uint32_t m0 = lds0 + (uint32_t)st * STAGE_B + (SPLIT ? 0u : (uint32_t)(wave * NKI) * 1024u);
+    const uint32_t m0 = lds0 + (uint32_t)st * STAGE_B + (uint32_t)(rb * NKI) * 1024u;
 #pragma unroll
     for (int k = 0; k < NKI; ++k) {
       dma16_s(kr, m0 + k * 1024u, koff[k], kso);
@@ -257,21 +278,28 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
 
   if (nl > 0) tile_load(tile_of(0), 0);
   wait_all_memory();
-  if constexpr (!SPLIT) __syncthreads();
+  if constexpr (SHARED) __syncthreads();
 
+  // Where a tile's body issues the next tile's loads. The tiled form at head
+  // dims above 64 does it behind the S product, whose operand reads they hold
+  // up otherwise (causal B=2 Hq=16 Hkv=4 S=4096 D=128 bf16 133.5 -> 127.9 us,
+  // D=96 -3%, non-causal within 1%). Narrower tiles and the other forms load
+  // first: their shorter steps leave later loads too little time to land (+2
+  // to +4%).
+  constexpr bool LATE = KG == 1 && DT > 64;
   // This wave's li-th tile on ring stage ST (a compile-time constant, so
   // every LDS offset in the body is an immediate).
   auto tile_body = [&](int li, auto stc) {
     constexpr int ST = decltype(stc)::value;
     if constexpr (NST == 2) {
-      if (li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
+      if (!LATE && li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
     }
     const int kbase = tile_of(li) * BN;
     // A causal tile whose first key is beyond every row of the wave is fully
     // masked for it. The split form's tiles all hold visible keys (its
     // ntiles ends at the block's last row), and its one-stage ring relies on
     // every tile body issuing the next tile's loads.
-    const bool active = SPLIT || !CAUSAL || kbase <= wq0 + QB * 32 - 1;
+    const bool active = !SHARED || ((KG == 1 || li < nl) && (!CAUSAL || kbase <= wq0 + QB * 32 - 1));
     if (active) {
       // S^T = K Q^T as a stream of 2 NKS MFMA slots (key block kb = m / NKS,
       // k-step ks = m % NKS); each slot also issues the LDS read of the
@@ -334,6 +362,9 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
       });
 
       __builtin_amdgcn_s_setprio(0);
+      if constexpr (LATE) {
+        if (li + 1 < nl) tile_load(tile_of(li + 1), ST ^ 1);
+      }
       if constexpr (NST == 1) {
         // Every K read of this tile fed an S product: the next K can land
         // while the softmax and the PV product run.
@@ -466,15 +497,15 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
     KF_WAIT_VMCNT(NST == 1 ? NKI : 0);
     // Every wave's loads landed; stage ST is free again. The split form's
     // rings are per wave, and the wave's own wait suffices.
-    if constexpr (!SPLIT) __syncthreads();
+    if constexpr (SHARED) __syncthreads();
   };
   if constexpr (NST == 2) {
-    for (int li = 0; li < nl; li += 2) {
+    for (int li = 0; li < nloop; li += 2) {
       tile_body(li, std::integral_constant<int, 0>{});
-      if (li + 1 < nl) tile_body(li + 1, std::integral_constant<int, 1>{});
+      if (li + 1 < nloop) tile_body(li + 1, std::integral_constant<int, 1>{});
     }
   } else {
-    for (int li = 0; li < nl; ++li) tile_body(li, std::integral_constant<int, 0>{});
+    for (int li = 0; li < nloop; ++li) tile_body(li, std::integral_constant<int, 0>{});
   }
 
   if constexpr (SPLIT) {
@@ -482,8 +513,8 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
     // overlays the other waves' rings, hence the barrier first.
     __syncthreads();
     float* ob = reinterpret_cast<float*>(smem);  // [wave][row][OSTR]
-    float* mb = ob + 4 * 32 * OSTR;              // [wave][row]
-    float* lb = mb + 4 * 32;                     // [wave][row]
+    float* mb = ob + NW * 32 * OSTR;             // [wave][row]
+    float* lb = mb + NW * 32;                    // [wave][row]
     {
       const float lt = wave_xor32_sum(l_i[0]);
       float* orow = ob + (wave * 32 + l32) * OSTR;
@@ -497,42 +528,42 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
       }
     }
     __syncthreads();
-    // Wave w stores head-dim columns [w DT/4, (w + 1) DT/4) of the 32 rows;
-    // a lane takes row l32 and half h32 of those columns.
-    constexpr int CW = DT / 4, CH = CW / 2;
+    // The KG waves of row block rb (waves rb + RB g) store its head-dim
+    // columns [kg DT/KG, (kg + 1) DT/KG); a lane takes row l32 and half h32 of
+    // those columns.
+    constexpr int CW = DT / KG, CH = CW / 2;
     static_assert(CH % 4 == 0, "stores are 4 columns wide");
-    const int row = l32;
-    float mw[4], M = kNegInf;
+    float mw[KG], M = kNegInf;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      mw[w] = mb[w * 32 + row];
-      M = fmaxf(M, mw[w]);
+    for (int g = 0; g < KG; ++g) {
+      mw[g] = mb[(rb + RB * g) * 32 + l32];
+      M = fmaxf(M, mw[g]);
     }
-    float sc[4], L = 0.f;
+    float sc[KG], L = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      // A wave with no tile (or only masked keys) for this row has m = -inf
+    for (int g = 0; g < KG; ++g) {
+      // A group with no tile (or only masked keys) for this row has m = -inf
       // and weight 0.
-      sc[w] = mw[w] == kNegInf ? 0.f : fast_exp2(mw[w] - M);
-      L += lb[w * 32 + row] * sc[w];
+      sc[g] = mw[g] == kNegInf ? 0.f : fast_exp2(mw[g] - M);
+      L += lb[(rb + RB * g) * 32 + l32] * sc[g];
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sc[w] *= inv;
-    const int qrow = q0 + row;
+    for (int g = 0; g < KG; ++g) sc[g] *= inv;
+    const int qrow = wq0 + l32;
     if (qrow < p.Sq) {
       uint16_t* Op = p.o + b * p.o_sb + h * p.o_sh + qrow * p.o_ss;
-      const int c0 = wave * CW + h32 * CH;
+      const int c0 = kg * CW + h32 * CH;
 #pragma unroll
       for (int j = 0; j < CH; j += 4) {
         const int d = c0 + j;
         if (d < p.D) {
           float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const float* src = ob + (w * 32 + row) * OSTR + d;
+          for (int g = 0; g < KG; ++g) {
+            const float* src = ob + ((rb + RB * g) * 32 + l32) * OSTR + d;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = fmaf(src[e], sc[w], o[e]);
+            for (int e = 0; e < 4; ++e) o[e] = fmaf(src[e], sc[g], o[e]);
           }
           u32x2 wv;
           wv[0] = pack2<T>(o[0], o[1]);
@@ -540,7 +571,7 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
           *reinterpret_cast<u32x2*>(Op + d) = wv;
         }
       }
-      if (wave == 0 && h32 == 0)
+      if (kg == 0 && h32 == 0)
         p.lse[((int64_t)b * p.Hq + h) * p.Sq + qrow] = L > 0.f ? (M + fast_log2(L)) * kLn2 : kNegInf;
     }
     return;
@@ -592,26 +623,35 @@ __global__ __launch_bounds__(256, ((QB == 1 && !SPLIT) ? (DT == 96 ? 3 : 2) : 1)
   }
 }
 
-template <typename T, int DT, int KS, int QB>
-static int launch_fwd(const FwdParams& prm, bool causal, hipStream_t stream) {
-  FwdParams p = prm;
-  const bool split = QB == 1 && attn_use_split(p.B, p.Hq, p.Sq, p.Sk, causal);
-  const int BM = split ? 32 : 4 * QB * 32;
-  p.nqt = cdiv(p.Sq, BM);
+template <typename T, int DT, int KS, int RB, int KG>
+static int launch_fwd_form(FwdParams p, bool causal, hipStream_t stream) {
+  p.nqt = cdiv(p.Sq, 32 * RB);
   const int64_t grid = (int64_t)p.nqt * p.B * p.Hq;
   if (grid > 0x7fffffff) return set_error(KF_EUNSUPPORTED, "kf_attn_fwd: grid too large");
-  const dim3 g((unsigned)grid), blk(256);
-  if (split) {
-    if (causal)
-      hipLaunchKernelGGL((fwd_kernel<T, DT, KS, 1, true, true>), g, blk, 0, stream, p);
-    else
-      hipLaunchKernelGGL((fwd_kernel<T, DT, KS, 1, false, true>), g, blk, 0, stream, p);
-  } else if (causal) {
-    hipLaunchKernelGGL((fwd_kernel<T, DT, KS, QB, true, false>), g, blk, 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((fwd_kernel<T, DT, KS, QB, false, false>), g, blk, 0, stream, p);
-  }
+  p.fold = fold_tiles(p.nqt, grid, fwd_waves_per_simd(DT, RB, KG) * 4 / (RB * KG));
+  const dim3 g((unsigned)grid), blk(64 * RB * KG);
+  if (causal)
+    hipLaunchKernelGGL((fwd_kernel<T, DT, KS, true, RB, KG>), g, blk, 0, stream, p);
+  else
+    hipLaunchKernelGGL((fwd_kernel<T, DT, KS, false, RB, KG>), g, blk, 0, stream, p);
   return check_launch("kf_attn_fwd");
+}
+
+template <typename T, int DT, int KS>
+static int launch_fwd(const FwdParams& p, bool causal, hipStream_t stream) {
+  switch (attn_form(kFwdCosts[DT / 32 - 1], p.B * p.Hq, p.Sq, p.Sk, causal)) {
+    case kForm4x2: return launch_fwd_form<T, DT, KS, 4, 2>(p, causal, stream);
+    case kForm2x2: return launch_fwd_form<T, DT, KS, 2, 2>(p, causal, stream);
+    case kForm2x4:
+      if constexpr (DT <= 64) return launch_fwd_form<T, DT, KS, 2, 4>(p, causal, stream);
+      break;
+    case kForm1x8:
+      if constexpr (DT == 64) return launch_fwd_form<T, DT, KS, 1, 8>(p, causal, stream);
+      break;
+    case kForm1x4: return launch_fwd_form<T, DT, KS, 1, 4>(p, causal, stream);
+    default: break;
+  }
+  return launch_fwd_form<T, DT, KS, 4, 1>(p, causal, stream);
 }
 
 template <typename T>
@@ -619,13 +659,13 @@ static int dispatch_fwd(const FwdParams& p, bool causal, hipStream_t stream) {
   // One 32-row block per wave at two waves per SIMD: while one wave runs its
   // softmax on the VALU the other keeps the MFMA pipe busy.
   switch (head_tile(p.D)) {
-    case 32: return launch_fwd<T, 32, 2, 1>(p, causal, stream);
-    case 64: return launch_fwd<T, 64, 4, 1>(p, causal, stream);
+    case 32: return launch_fwd<T, 32, 2>(p, causal, stream);
+    case 64: return launch_fwd<T, 64, 4>(p, causal, stream);
     case 96:
       // Head dims 72 and 80 end 16 columns before the tile does.
-      return p.D <= 80 ? launch_fwd<T, 96, 5, 1>(p, causal, stream)
-                       : launch_fwd<T, 96, 6, 1>(p, causal, stream);
-    default: return launch_fwd<T, 128, 8, 1>(p, causal, stream);
+      return p.D <= 80 ? launch_fwd<T, 96, 5>(p, causal, stream)
+                       : launch_fwd<T, 96, 6>(p, causal, stream);
+    default: return launch_fwd<T, 128, 8>(p, causal, stream);
   }
 }
 

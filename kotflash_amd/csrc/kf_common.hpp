@@ -357,6 +357,20 @@ template <> __device__ inline float sum2_acc<__bf16>(uint32_t x, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x), one, acc, false);
 }
 
+// Dispatch order of causal query tiles when the whole grid is resident at
+// once: the j-th of n workgroups (per_round of which fill one workgroup slot
+// of every CU) takes the tile of this rank in the longest-first order. Every
+// second round of slots is filled in reverse, so that a CU's first long tile
+// shares it with a short one.
+// `on` (0 or 1) turns it off without a branch: a branch here would split the
+// kernel-argument loads into several cold round trips.
+template <int PER_ROUND>
+__device__ inline int fold_rank(int j, int n, int on) {
+  const int r = j / PER_ROUND;
+  const int ends = 2 * r * PER_ROUND + min(PER_ROUND, n - r * PER_ROUND) - 1;  // first + last of the round
+  return (r & on) ? ends - j : j;
+}
+
 __host__ __device__ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace kf

@@ -27,21 +27,113 @@ inline int head_tile(int64_t D) {
   return 128;
 }
 
-// The split forms of the forward and dQ kernels (32-row workgroups whose
-// waves split the key range) run when a grid of 128-row tiles would leave
-// most of the 256 CUs idle and a tile sees more than two K/V tiles: config
-// 1's 64 workgroups, for instance, become 256 with chains of at most two
-// tiles. The split grid (four times the tiles, one workgroup per CU) fits
-// one round of the CUs up to 64 tiles; causal grids, whose tiles differ in
-// length, still gain up to 128. Measured on MI355X for the forward against
-// the tiled form: config 1 -37%; 256 tiles, or non-causal D >= 96 at 96-128
-// tiles, 5-20% slower split.
-constexpr int64_t kSplitMaxTiles = 64;
-constexpr int64_t kSplitMaxTilesCausal = 128;
+// Forms of the forward and dQ kernels: RB row blocks of 32 query rows times KG
+// key groups, RB * KG waves per workgroup. A group's waves take every KG-th
+// K/V tile of the workgroup's rows, and the groups' results are combined
+// through LDS at the end. 4x1 moves the fewest K/V bytes per product and
+// is the one for large problems; with few tiles the launch is as long as its
+// longest chain of dependent tiles, and splitting the keys (and the rows into
+// more workgroups) shortens it.
+enum AttnForm { kForm4x1, kForm4x2, kForm2x2, kForm2x4, kForm1x4, kForm1x8, kNumForms };
+struct FormShape {
+  int rb, kg;
+};
+constexpr FormShape kFormShapes[kNumForms] = {{4, 1}, {4, 2}, {2, 2}, {2, 4}, {1, 4}, {1, 8}};
 
-inline bool attn_use_split(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, bool causal) {
-  const int64_t tiles = (Sq + 127) / 128 * B * Hq;
-  return Sk > 128 && tiles <= (causal ? kSplitMaxTilesCausal : kSplitMaxTiles);
+// Launch time of a form, us: `fixed` once, `round` for each round of workgroup
+// slots (256 CUs times per_cu), and the K/V steps: a workgroup's step of 64
+// keys per group takes `chain` when it has its CU to itself, and a CU retires
+// one per `work` when several share it.
+struct FormCost {
+  float fixed, round, chain, work;
+  int per_cu;  // resident workgroups per CU; 0: the form is not built
+};
+
+// Fitted to 580 shapes on MI355X (1 to 32 heads, batches of 1 to 16, 45 to
+// 4096 queries, 45 to 6600 keys, up to 1024 tiles; rms error 3 to 14%).
+constexpr FormCost kFwdCosts[4][kNumForms] = {  // by head-dim tile / 32 - 1; forms as in AttnForm
+    {{3.39f, 0.00f, 0.58f, 0.44f, 2}, {0.90f, 2.98f, 0.83f, 0.87f, 1}, {3.38f, 0.28f, 0.59f, 0.46f, 2},
+     {1.21f, 2.63f, 0.91f, 0.91f, 1}, {3.08f, 0.72f, 0.46f, 0.45f, 1}, {0, 0, 0, 0, 0}},
+    {{4.19f, 0.00f, 0.70f, 0.59f, 2}, {0.00f, 5.05f, 1.02f, 1.07f, 1}, {0.04f, 4.21f, 0.79f, 0.59f, 2},
+     {0.47f, 4.22f, 1.17f, 1.22f, 1}, {1.25f, 2.63f, 0.87f, 0.87f, 1}, {0.84f, 3.33f, 1.32f, 1.32f, 1}},
+    {{0.00f, 4.62f, 0.84f, 0.85f, 3}, {0.00f, 5.53f, 1.16f, 1.31f, 1}, {0.85f, 3.68f, 1.01f, 1.05f, 1},
+     {0, 0, 0, 0, 0}, {1.34f, 3.13f, 1.05f, 1.07f, 1}, {0, 0, 0, 0, 0}},
+    {{0.00f, 5.13f, 1.06f, 1.08f, 2}, {0.00f, 6.74f, 1.43f, 1.77f, 1}, {0.00f, 5.28f, 1.17f, 1.36f, 1},
+     {0, 0, 0, 0, 0}, {0.89f, 3.64f, 1.40f, 1.42f, 1}, {0, 0, 0, 0, 0}},
+};
+constexpr FormCost kDqCosts[4][kNumForms] = {  // by head-dim tile / 32 - 1; forms as in AttnForm
+    {{3.72f, 0.21f, 0.56f, 0.44f, 2}, {0.78f, 3.54f, 0.77f, 0.85f, 1}, {2.46f, 1.68f, 0.58f, 0.44f, 2},
+     {0.98f, 3.18f, 0.89f, 0.94f, 1}, {3.07f, 0.82f, 0.51f, 0.51f, 1}, {0, 0, 0, 0, 0}},
+    {{0.00f, 5.09f, 0.75f, 0.81f, 2}, {0.00f, 6.25f, 1.19f, 1.33f, 1}, {0.19f, 5.15f, 0.85f, 0.79f, 2},
+     {0.69f, 5.48f, 1.40f, 1.42f, 1}, {1.11f, 3.91f, 0.87f, 0.90f, 1}, {0.97f, 4.54f, 1.57f, 1.58f, 1}},
+    {{0.00f, 4.69f, 0.94f, 1.03f, 2}, {0.00f, 6.12f, 1.44f, 1.79f, 1}, {0.43f, 4.69f, 1.11f, 1.17f, 1},
+     {0, 0, 0, 0, 0}, {0.85f, 3.89f, 1.41f, 1.38f, 1}, {0, 0, 0, 0, 0}},
+    {{0.00f, 6.97f, 1.32f, 1.34f, 2}, {0.00f, 9.65f, 2.06f, 2.58f, 1}, {0.00f, 7.17f, 1.47f, 1.58f, 1},
+     {0, 0, 0, 0, 0}, {0.95f, 5.68f, 1.59f, 1.77f, 1}, {0, 0, 0, 0, 0}},
+};
+
+inline float attn_form_cost(const FormCost& c, const FormShape& f, int64_t heads, int64_t Sq, int64_t Sk,
+                            bool causal) {
+  const int rows = 32 * f.rb, keys = 64 * f.kg;
+  const int64_t tiles = (Sq + rows - 1) / rows;
+  const int64_t longest = causal && tiles * rows < Sk ? tiles * rows : Sk;
+  const int64_t top = (longest + keys - 1) / keys;  // steps of the longest tile
+  const int64_t wgs = tiles * heads, slots = 256 * c.per_cu;
+  if (!causal) {
+    // Equal workgroups: whole rounds, the last one perhaps with fewer per CU.
+    const int64_t rest = wgs % slots;
+    const float alone = top * c.chain, shared = top * c.work;
+    float t = c.fixed + (wgs / slots) * (c.round + (alone > c.per_cu * shared ? alone : c.per_cu * shared));
+    if (rest) {
+      const float last = shared * ((rest + 255) / 256);
+      t += c.round + (alone > last ? alone : last);
+    }
+    return t;
+  }
+  // Causal tile q sees min(Sk, (q + 1) rows) keys: those before tile m,
+  // growing, then Sk (half a step on average for the last, partly filled one).
+  // Unequal workgroups, longest first, fill in for one another.
+  const float m = (float)(tiles < Sk / rows ? tiles : Sk / rows);
+  const float steps = (rows * m * (m + 1.f) / 2.f + (tiles - m) * Sk) / keys + (f.kg > 1 || f.rb < 2 ? 0.5f * m : 0.f);
+  const float rounds = (float)wgs / slots;
+  const float chain = top * c.chain, work = steps * heads / 256.f * c.work;
+  return c.fixed + c.round * (rounds > 1.f ? rounds : 1.f) + (chain > work ? chain : work);
+}
+
+// The form of a problem. The default is 1x4 for grids of 128-row tiles that
+// leave most of the 256 CUs idle (at most 64 tiles, 128 when causal, whose
+// tiles differ in length) and 4x1 for the others; another form is taken when
+// the costs above make it at least 8% faster, a margin that covers most of
+// their error. Over the 580 shapes this took the forward 5% and dQ 7% off the
+// default time in the geometric mean (up to 54%: dQ, B=4 H=8 Sq=300 Sk=1500
+// D=128, 58.9 -> 26.8 us); of the 162 that changed form 2 got more than 4%
+// slower (6% at most).
+constexpr int64_t kFormMaxTiles = 512;  // past two 4x1 workgroups per CU other forms lost 5-18%
+
+inline AttnForm attn_form(const FormCost (&costs)[kNumForms], int64_t heads, int64_t Sq, int64_t Sk, bool causal) {
+  const int64_t tiles = (Sq + 127) / 128 * heads;
+  if (tiles > kFormMaxTiles) return kForm4x1;
+  int best = Sk > 128 && tiles <= (causal ? 128 : 64) ? kForm1x4 : kForm4x1;
+  float least = 0.92f * attn_form_cost(costs[best], kFormShapes[best], heads, Sq, Sk, causal);
+  for (int f = 0; f < kNumForms; ++f) {
+    if (costs[f].per_cu == 0) continue;
+    const float t = attn_form_cost(costs[f], kFormShapes[f], heads, Sq, Sk, causal);
+    if (t < least) {
+      least = t;
+      best = f;
+    }
+  }
+  return (AttnForm)best;
+}
+
+// Whether a causal grid takes its tiles in fold_rank's order: when all its
+// workgroups are resident at once, in more than one per CU, so that the
+// pairing on a CU is decided by the order alone, and the tiles of a head
+// differ enough in length. Measured (tiled form, forward / dQ): B=1 Hq=32
+// Hkv=8 S=1777 D=128 bf16 -6.7% / -4.2%, B=1 Hq=16 S=4096 D=64 dQ -5.8%, four
+// tiles per head (B=8 Hq=12 S=386 D=128) +6%.
+inline int fold_tiles(int64_t tiles_per_head, int64_t grid, int per_cu) {
+  return tiles_per_head >= 8 && grid > 256 && grid <= 256 * per_cu;
 }
 
 }  // namespace kf
