@@ -1274,7 +1274,33 @@ __global__ __launch_bounds__(256) void dkdv_fixup_kernel(const BwdParams p, cons
     const int kr = sub * kFixKeys + e / QPR, d = (e % QPR) * 4;
     if (d >= p.D) continue;
     float4 sk = make_float4(0.f, 0.f, 0.f, 0.f), sv = sk;
-    for (int w = w0; w <= w1; ++w) {
+    int w = w0;
+    // Rows in many shares (grouped heads, few tiles): four shares' loads at a
+    // time, added in the same order; one after the other they cost a memory
+    // latency each (dK/dV and fixup at B=1 Hq=8 Hkv=1 S=700 D=96, 43 shares a
+    // row: 72.4 -> 41.1 us; B=2 Hq=8 Hkv=2 S=1024 D=64 causal 33.6 -> 28.6; two
+    // shares a row unchanged). An empty share reads share w0's slot (never
+    // empty) and adds nothing.
+    for (; w + 3 <= w1; w += 4) {
+      float4 a[4], c[4];
+      bool some[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        some[j] = sp.start[w + j + 1] != sp.start[w + j];
+        const int x = some[j] ? w + j : w0;
+        const int side = sp.start[x] >= first ? 0 : 1;
+        const float* slot = p.part + (2 * x + side) * 2 * kBNK * DT + (int64_t)kr * DT + d;
+        a[j] = *reinterpret_cast<const float4*>(slot);
+        c[j] = *reinterpret_cast<const float4*>(slot + kBNK * DT);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (!some[j]) continue;
+        sk.x += a[j].x; sk.y += a[j].y; sk.z += a[j].z; sk.w += a[j].w;
+        sv.x += c[j].x; sv.y += c[j].y; sv.z += c[j].z; sv.w += c[j].w;
+      }
+    }
+    for (; w <= w1; ++w) {
       const int64_t wu0 = sp.start[w];
       if (sp.start[w + 1] == wu0) continue;  // empty share: wrote nothing
       const int side = wu0 >= first ? 0 : 1;
@@ -1315,6 +1341,21 @@ static int dkdv_workgroups() {
   return n < kMaxDkdvWG ? n : kMaxDkdvWG;
 }
 
+// Shares of a problem: one per CU, or fewer where they would hold less than
+// kMinShareUnits units each: a share then costs more in its segment starts and
+// in the fp32 partials that the fixup sums (one per share and row it touches)
+// than its units take. A multiple of 8, for the XCD mapping. Measured over
+// twelve small shapes, us for dK/dV and fixup, one share per CU -> 4 -> 8
+// units: B=1 Hq=8 Hkv=1 S=700 D=96 41.2 -> 33.0 -> 27.4, B=2 Hq=8 Hkv=2 S=1024
+// D=64 causal 28.6 -> 28.4 -> 24.3, B=2 Hq=8 Hkv=2 S=512 D=64 causal 22.9 ->
+// 19.2 -> 20.6; 8 is 4% ahead of 4 in the geometric mean.
+constexpr int kMinShareUnits = 8;
+static int dkdv_share_count(int nwg, int64_t units, int64_t rows) {
+  // Not below one share per tile row: whole rows cost no partials.
+  const int64_t n = ((units / kMinShareUnits > rows ? units / kMinShareUnits : rows) + 7) / 8 * 8;
+  return n < 8 ? (nwg < 8 ? nwg : 8) : n < nwg ? (int)n : nwg;
+}
+
 static size_t delta_bytes(int64_t B, int64_t Hq, int64_t Sq) {
   return ((size_t)B * Hq * Sq * sizeof(float) + 255) / 256 * 256;
 }
@@ -1326,15 +1367,27 @@ static size_t delta_bytes(int64_t B, int64_t Hq, int64_t Sq) {
 // 1-2% slower than 5. With the long-short tile order and cuts charged to the
 // share that makes them, 3, 7 and 10 units were 0.4-1.2% slower than 5.
 constexpr int kSegmentCost8 = 40;
+// Cut tile rows also cost their fp32 partials, stored by the dK/dV launch and
+// summed by a fixup launch of its own. Shares of whole consecutive rows cost
+// neither, and are taken when that leaves the longest share no more than this
+// (8ths of a unit, by head-dim tile / 32 - 1) above an even one. Measured, us
+// for dK/dV and fixup, cut -> whole rows: B=4 H=12 S=1000 D=64 causal 41.4 ->
+// 27.9 (longest share 26.1 units against 21.0), B=4 H=16 S=512 D=128 causal
+// 39.4 -> 24.1 (13.0, 10.0), B=4 H=12 S=2048 D=64 causal 90.7 -> 76.7 (81.2,
+// 66.0), B=1 H=8 S=2000 D=128 52.3 -> 64.3 (37.4, 18.5). Over 19 shapes the cuts
+// cost 11 to 31 units at D = 128 and 14 to 32 at D = 64.
+constexpr int kFixupCost8[4] = {112, 112, 104, 88};
+constexpr int kMaxWholeRows = 1024;
 // Returns the number of tile rows that a share boundary cuts (shared tiles).
-static int dkdv_split(DkdvSplit& sp, int ngroups, int G, int nqt, int nkt, bool causal, int nwg) {
+// `fixup8`: what cuts cost besides their segment starts (kFixupCost8).
+static int dkdv_split(DkdvSplit& sp, int ngroups, int G, int nqt, int nkt, bool causal, int nwg, int fixup8) {
   struct Key {
-    int ngroups, G, nqt, nkt, causal, nwg;
+    int ngroups, G, nqt, nkt, causal, nwg, fixup8;
   };
-  thread_local Key last{-1, 0, 0, 0, 0, 0};
+  thread_local Key last{-1, 0, 0, 0, 0, 0, 0};
   thread_local DkdvSplit cached;
   thread_local int cached_shared = 0;
-  const Key k{ngroups, G, nqt, nkt, causal ? 1 : 0, nwg};
+  const Key k{ngroups, G, nqt, nkt, causal ? 1 : 0, nwg, fixup8};
   if (memcmp(&k, &last, sizeof k) != 0) {
     int64_t rows_cost = 0, all_units = 0;
     for (int kt = 0; kt < nkt; ++kt) {
@@ -1396,6 +1449,43 @@ static int dkdv_split(DkdvSplit& sp, int ngroups, int G, int nqt, int nkt, bool 
       }
       cuts = rcuts;
     }
+    // Shares of whole rows, the longest of them as short as consecutive rows
+    // allow: a bound on a share's cost is feasible if filling shares up to it
+    // needs no more than nwg of them.
+    const int rows = ngroups * mseen;
+    if (shared > 0 && mseen == nkt && rows <= kMaxWholeRows) {
+      auto pack = [&](DkdvSplit& out, int64_t bound) {
+        int w = 0;
+        int64_t base = 0, in = 0;
+        out.start[0] = 0;
+        for (int g = 0; g < ngroups; ++g)
+          for (int pos = 0; pos < nkt; ++pos) {
+            const int64_t units = (int64_t)G * dkdv_nq(dkdv_tile_at(pos, mseen), nqt, causal);
+            const int64_t c = 8 * units + kSegmentCost8;
+            if (c > bound) return false;
+            if (in + c > bound) {
+              if (++w == nwg) return false;
+              out.start[w] = (int)base;
+              in = 0;
+            }
+            in += c;
+            base += units;
+          }
+        while (++w <= nwg) out.start[w] = (int)all_units;
+        return true;
+      };
+      int64_t lo = rows_cost / nwg, hi = lo + fixup8;
+      DkdvSplit whole;
+      if (pack(whole, hi)) {
+        shared = 0;
+        while (hi - lo > 8) {
+          cached = whole;
+          const int64_t mid = (lo + hi) / 2;
+          if (pack(whole, mid)) hi = mid; else { lo = mid; whole = cached; }
+        }
+        cached = whole;
+      }
+    }
     cached_shared = shared;
     last = k;
   }
@@ -1449,9 +1539,10 @@ static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) 
     p.nqt = cdiv(p.Sq, kBMQ);
     p.nkt = cdiv(p.Sk, kBNK);
     p.units = dkdv_total_units(p.ngroups, p.G, p.nqt, p.nkt, causal);
+    p.nwg = dkdv_share_count(p.nwg, p.units, (int64_t)p.ngroups * dkdv_seen_tiles(p.nqt, p.nkt, causal));
     if (p.units > 0x7fffffff) return set_error(KF_EINVAL, "kf_attn_bwd: problem too large for one dK/dV launch");
     DkdvSplit sp;
-    dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg);
+    dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg, kFixupCost8[DT / 32 - 1]);
     if (causal)
       hipLaunchKernelGGL((dkdv_kernel<T, DT, KS, true>), dim3((unsigned)p.nwg), dim3(256), 0, stream, p, sp);
     else
@@ -1463,8 +1554,9 @@ static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) 
     p.nqt = cdiv(p.Sq, kBMQ);
     p.nkt = cdiv(p.Sk, kBNK);
     p.units = dkdv_total_units(p.ngroups, p.G, p.nqt, p.nkt, causal);
+    p.nwg = dkdv_share_count(p.nwg, p.units, (int64_t)p.ngroups * dkdv_seen_tiles(p.nqt, p.nkt, causal));
     DkdvSplit sp;
-    const int shared = dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg);
+    const int shared = dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg, kFixupCost8[DT / 32 - 1]);
     const int64_t unseen = (int64_t)p.ngroups * (p.nkt - dkdv_seen_tiles(p.nqt, p.nkt, causal));
     if (shared > 0 || unseen > 0) {
       const int64_t grid = (int64_t)p.nkt * p.ngroups * kFixSub;
