@@ -309,6 +309,13 @@ class RaggedKVCache(PreallocatedKVCache):
                  else torch.cuda.ExternalStream(self._writer, device=dev))
         torch.cuda.current_stream(dev).wait_stream(other)
 
+    def __getstate__(self):
+        """For copy and pickle: the stream handle means nothing in another
+        process, so the current stream waits here, before the tensors are
+        read, and the copy starts without one."""
+        self._order_streams()
+        return {name: x for name, x in self.__dict__.items() if name != "_writer"}
+
     def _set(self, lengths: List[int], wait: bool = True) -> None:
         """Set the lengths on the host and in the device mirrors. ``wait``:
         return once the mirrors are written, whatever stream reads them next;
@@ -420,6 +427,7 @@ class RaggedKVCache(PreallocatedKVCache):
 
     def view(self, b: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
         """Storage-backed [1, Hkv, lengths[b], D] views of sequence b."""
+        self._order_streams()
         if self.lengths[b] == 0:
             raise ValueError("KV cache is empty")
         n = self.lengths[b]

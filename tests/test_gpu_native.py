@@ -1,6 +1,9 @@
 """The C++ launch path (kotflash_amd._native) against the Python path it
 stands in for: the same bits for every form both accept, the same refusals,
 and autograd's hooks, checkpointing and streams as with a Python Function."""
+import copy
+import pickle
+
 import pytest
 import torch
 from torch.utils.checkpoint import checkpoint
@@ -172,3 +175,23 @@ def test_ragged_lengths_across_streams():
     assert lens.tolist() == cache.lengths == [i % 50 + 2 for i in range(b)]
     assert torch.equal(got, cache.attend(q))
     assert cache.starts.tolist() == cache.lengths
+
+
+def test_ragged_copies_carry_no_stream():
+    """A copied or unpickled cache holds the appended tokens and lengths, and
+    no handle of the stream that wrote them."""
+    cache = RaggedKVCache(2, 1, 1200, 64, device="cuda", dtype=F16)
+    cache.k.copy_(seeded((2, 1, 1200, 64), 93, dtype=F16))
+    cache.v.copy_(seeded((2, 1, 1200, 64), 94, dtype=F16))
+    cache.set_lengths([5, 1100])
+    side = torch.cuda.Stream()
+    new = [seeded((2, 1, 3, 64), 95 + i, dtype=F16) for i in range(2)]
+    q = seeded((2, 1, 1, 64), 97, dtype=F16)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        cache.append(*new)
+    assert cache._writer is not None
+    for other in (copy.deepcopy(cache), pickle.loads(pickle.dumps(cache))):
+        assert other._writer is None and other.lengths == cache.lengths
+        assert other.seqlens.tolist() == other.starts.tolist() == [8, 1103]
+        assert torch.equal(other.attend(q), cache.attend(q))
