@@ -293,51 +293,21 @@ class RaggedKVCache(PreallocatedKVCache):
             raise ValueError(f"lengths must be in [0, max_len={self.max_len}]")
         self._set(lengths)
 
-    # Stream (raw handle) of the last append, whose tokens and lengths a call
-    # on another stream has to wait for; None when the host has waited.
-    _writer = None
-
-    def _order_streams(self) -> None:
-        """Make the current stream wait for the last append if that ran on
-        another one. (Under graph capture nothing may be waited for; starting
-        a capture synchronizes with the device.)"""
-        if self._writer is None or _hip._stream(self.k.device) == self._writer \
-                or torch.cuda.is_current_stream_capturing():
-            return
-        dev = self.k.device
-        other = (torch.cuda.default_stream(dev) if self._writer == 0
-                 else torch.cuda.ExternalStream(self._writer, device=dev))
-        torch.cuda.current_stream(dev).wait_stream(other)
-
-    def __getstate__(self):
-        """For copy and pickle: the stream handle means nothing in another
-        process, so the current stream waits here, before the tensors are
-        read, and the copy starts without one."""
-        self._order_streams()
-        return {name: x for name, x in self.__dict__.items() if name != "_writer"}
-
-    def _set(self, lengths: List[int], wait: bool = True) -> None:
-        """Set the lengths on the host and in the device mirrors. ``wait``:
-        return once the mirrors are written, whatever stream reads them next;
-        an append (``wait=False``) only orders them after its own writes, on
-        its stream."""
+    def _set(self, lengths: List[int]) -> None:
+        """Set the lengths on the host and in the device mirrors. Returns once
+        the current stream has written them, and with them everything queued
+        there before: an append's tokens, lengths and output may be read on
+        any stream next, by any tensor that shares their memory, or freed."""
         self.lengths = lengths
         self.length = max(lengths) if lengths else 0
         if not torch.compiler.is_compiling() \
                 and _hip.native().store_lengths(self.starts, self.seqlens, lengths) is None:
-            if wait:
-                torch.cuda.current_stream(self.k.device).synchronize()
-                self._writer = None
-            else:
-                self._writer = _hip._stream(self.k.device)
             return
-        self._writer = None
         host = torch.tensor(lengths, dtype=torch.int64)
         self.starts.copy_(host, non_blocking=False)
         self.seqlens.copy_(host.to(torch.int32), non_blocking=False)
 
     def append(self, new_k: torch.Tensor, new_v: torch.Tensor, *, backend: str = "auto") -> None:
-        self._order_streams()
         self._check_new(new_k, new_v)
         if backend not in APPEND_BACKENDS:
             raise ValueError("append backend must be one of: auto, torch, hip or cuda")
@@ -357,7 +327,7 @@ class RaggedKVCache(PreallocatedKVCache):
             for b, start in enumerate(self.lengths):
                 self.k[b, :, start:start + n].copy_(new_k[b])
                 self.v[b, :, start:start + n].copy_(new_v[b])
-        self._set([x + n for x in self.lengths], wait=False)
+        self._set([x + n for x in self.lengths])
 
     def append_and_attend(self, q_new, new_k, new_v, *, append_backend: str = "auto",
                           attention_backend: str = "auto") -> torch.Tensor:
@@ -371,7 +341,6 @@ class RaggedKVCache(PreallocatedKVCache):
         otherwise it appends (``append``) and attends (``attend``) as two
         steps.
         """
-        self._order_streams()
         if (_fuses_plainly(self, q_new, new_k, new_v, append_backend, attention_backend)
                 and max(self.lengths) + new_k.shape[2] <= self.max_len):
             from .kernels import hip_decode
@@ -381,7 +350,7 @@ class RaggedKVCache(PreallocatedKVCache):
                 q_new, self.k, self.v, new_k, new_v, self.seqlens, host_lengths=self.lengths,
                 scale=1.0 / (q_new.shape[-1] ** 0.5),
             )
-            self._set([x + n for x in self.lengths], wait=False)
+            self._set([x + n for x in self.lengths])
             return out
         if attention_backend not in ("auto", "hip", "triton", "sdpa"):
             raise ValueError("attention backend must be one of: auto, hip, triton or sdpa")
@@ -420,14 +389,13 @@ class RaggedKVCache(PreallocatedKVCache):
                 q_new, self.k, self.v, new_k, new_v, self.seqlens, host_lengths=self.lengths,
                 scale=1.0 / (q_new.shape[-1] ** 0.5),
             )
-            self._set([x + n for x in self.lengths], wait=False)
+            self._set([x + n for x in self.lengths])
             return out
         self.append(new_k, new_v, backend=append_backend)
         return self.attend(q_new, backend=attention_backend)
 
     def view(self, b: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
         """Storage-backed [1, Hkv, lengths[b], D] views of sequence b."""
-        self._order_streams()
         if self.lengths[b] == 0:
             raise ValueError("KV cache is empty")
         n = self.lengths[b]
@@ -437,7 +405,6 @@ class RaggedKVCache(PreallocatedKVCache):
         """Non-causal decode of q [B, Hq, Sq, D]; rows of sequence b see its
         first lengths[b] positions. HIP: one split-KV decode launch for all
         sequences; SDPA: one call per sequence."""
-        self._order_streams()
         if not isinstance(q, torch.Tensor) or q.ndim != 4:
             raise ValueError("q must use [B, Hq, Sq, D] layout")
         if q.shape[0] != self.k.shape[0] or q.shape[-1] != self.k.shape[-1]:

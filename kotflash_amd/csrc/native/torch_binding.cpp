@@ -438,8 +438,9 @@ PyObject* py_step_args(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // store_lengths(starts, seqlens, lengths): the host lengths into a ragged
 // cache's int64 and int32 device arrays, one launch that carries them by value
-// instead of two copies that wait for the stream. Not under graph capture,
-// where a replay would repeat these values.
+// instead of two copies. Like a copy from pageable memory it returns when the
+// stream has done it: the cache's tensors may then be read on any stream. Not
+// under graph capture, where a replay would repeat these values.
 PyObject* py_store_lengths(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   std::vector<int32_t> lens;
@@ -459,8 +460,12 @@ PyObject* py_store_lengths(PyObject*, PyObject* const* args, Py_ssize_t n) {
     (void)hipGetLastError();
     return not_handled();
   }
-  check(kf_store_lengths(starts->data_ptr<int64_t>(), seqlens->data_ptr<int32_t>(), lens.data(), count, stream),
-        "kf_store_lengths");
+  {
+    pybind11::gil_scoped_release nogil;
+    check(kf_store_lengths(starts->data_ptr<int64_t>(), seqlens->data_ptr<int32_t>(), lens.data(), count, stream),
+          "kf_store_lengths");
+    c10::hip::getCurrentHIPStream(starts->device().index()).synchronize();
+  }
   starts->unsafeGetTensorImpl()->bump_version();
   seqlens->unsafeGetTensorImpl()->bump_version();
   Py_RETURN_NONE;

@@ -156,14 +156,21 @@ def test_cache_steps_match_the_python_path(python_path, kind):
         assert torch.equal(a, e), i
 
 
+def _ragged(b, cap, lengths, dtype=F16):
+    cache = RaggedKVCache(b, 1, cap, 64, device="cuda", dtype=dtype)
+    cache.k.copy_(seeded((b, 1, cap, 64), 93, dtype=dtype))
+    cache.v.copy_(seeded((b, 1, cap, 64), 94, dtype=dtype))
+    cache.set_lengths(lengths)
+    return cache
+
+
 def test_ragged_lengths_across_streams():
-    """A step on another stream waits for the last append's tokens and
-    lengths; set_lengths returns with the mirrors written."""
-    b, hkv, cap, d = 300, 1, 64, 64  # two launches of the lengths kernel
-    cache = RaggedKVCache(b, hkv, cap, d, device="cuda", dtype=F16)
-    cache.set_lengths([i % 50 for i in range(b)])
-    new = [seeded((b, hkv, 2, d), 90 + i, dtype=F16) for i in range(2)]
-    q = seeded((b, 1, 1, d), 92, dtype=F16)
+    """A step on another stream finds the last append's tokens and lengths;
+    set_lengths returns with the mirrors written."""
+    b, cap = 300, 64  # two launches of the lengths kernel
+    cache = _ragged(b, cap, [i % 50 for i in range(b)])
+    new = [seeded((b, 1, 2, 64), 90 + i, dtype=F16) for i in range(2)]
+    q = seeded((b, 1, 1, 64), 92, dtype=F16)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     torch.cuda._sleep(20_000_000)
@@ -173,25 +180,50 @@ def test_ragged_lengths_across_streams():
         lens = cache.seqlens.clone()
     torch.cuda.synchronize()
     assert lens.tolist() == cache.lengths == [i % 50 + 2 for i in range(b)]
-    assert torch.equal(got, cache.attend(q))
+    assert torch.isfinite(got).all() and torch.equal(got, cache.attend(q))
     assert cache.starts.tolist() == cache.lengths
 
 
+@pytest.mark.parametrize("fused", [False, True])
+def test_ragged_append_returns_with_its_work_done(fused):
+    """An append behind queued work of its stream: whatever another stream
+    does next, without a wait of its own, sees the append's tokens, lengths and
+    output, and lengths set from there stay set."""
+    b, cap, lengths = 3, 1200, [0, 1100, 700]
+    cache = _ragged(b, cap, lengths)
+    new = [seeded((b, 1, 3, 64), 95 + i, dtype=F16) for i in range(2)]
+    q = seeded((b, 4, 3, 64), 97, dtype=F16)
+    held = cache.k[:, :, :], cache.seqlens[:], cache.starts[:]  # taken before the append
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)
+        out = cache.append_and_attend(q, *new) if fused else cache.append(*new)
+    k, seqlens, starts = (t.clone() for t in held)
+    got = out.clone() if fused else None
+    cache.set_lengths(lengths)  # drop the tokens again, from this stream
+    torch.cuda.synchronize()
+    assert seqlens.tolist() == starts.tolist() == [x + 3 for x in lengths]
+    for i, n in enumerate(lengths):
+        assert torch.equal(k[i, :, n:n + 3], new[0][i])
+    assert cache.seqlens.tolist() == cache.starts.tolist() == cache.lengths == lengths
+    if fused:
+        again = cache.append_and_attend(q, *new)
+        assert torch.isfinite(got).all() and torch.equal(got, again)
+
+
 def test_ragged_copies_carry_no_stream():
-    """A copied or unpickled cache holds the appended tokens and lengths, and
-    no handle of the stream that wrote them."""
-    cache = RaggedKVCache(2, 1, 1200, 64, device="cuda", dtype=F16)
-    cache.k.copy_(seeded((2, 1, 1200, 64), 93, dtype=F16))
-    cache.v.copy_(seeded((2, 1, 1200, 64), 94, dtype=F16))
-    cache.set_lengths([5, 1100])
+    """A copied or unpickled cache holds the tokens and lengths appended on
+    another stream."""
+    cache = _ragged(2, 1200, [5, 1100])
     side = torch.cuda.Stream()
     new = [seeded((2, 1, 3, 64), 95 + i, dtype=F16) for i in range(2)]
     q = seeded((2, 1, 1, 64), 97, dtype=F16)
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)
         cache.append(*new)
-    assert cache._writer is not None
-    for other in (copy.deepcopy(cache), pickle.loads(pickle.dumps(cache))):
-        assert other._writer is None and other.lengths == cache.lengths
+    for other in (copy.copy(cache), copy.deepcopy(cache), pickle.loads(pickle.dumps(cache))):
+        assert other.lengths == cache.lengths
         assert other.seqlens.tolist() == other.starts.tolist() == [8, 1103]
         assert torch.equal(other.attend(q), cache.attend(q))
