@@ -12,6 +12,7 @@ the library is missing or a call fails, a RuntimeError is raised.
 from __future__ import annotations
 
 import ctypes
+import warnings
 from functools import lru_cache
 from pathlib import Path
 from typing import Optional
@@ -79,18 +80,13 @@ def lib() -> ctypes.CDLL:
     version = handle.kf_abi_version()
     if version != ABI_VERSION:
         raise RuntimeError(f"kotflash_amd ABI mismatch: library {version}, bindings {ABI_VERSION}")
-    try:
-        from . import _native  # noqa: F401
-    except ImportError as exc:
-        raise RuntimeError(f"kotflash_amd native module not usable ({exc}); build it with "
-                           "`python -m kotflash_amd.build`") from exc
     return handle
 
 
 class _NoNative:
-    """Stands in for the native module where it is not built: every call is
-    left to the Python path (which raises on a GPU, where the library is
-    missing too)."""
+    """Stands in for the native module where it does not load: every call is
+    left to the Python path, which runs the same kernels through ctypes (and
+    raises on a GPU where the library is missing too)."""
 
     def __getattr__(self, name):
         return _not_handled
@@ -106,13 +102,19 @@ _NATIVE = None
 def native():
     """``kotflash_amd._native``, the C++ launch path (csrc/native). Its entries
     return NotImplemented, before doing anything, for calls that are not the
-    ordinary case."""
+    ordinary case. A module that does not load (built for another torch or
+    Python) costs host time only, and is reported once."""
     global _NATIVE
     if _NATIVE is None:
         if not library_available():
             return _NoNative()
-        from . import _native
-
+        try:
+            from . import _native
+        except ImportError as exc:
+            warnings.warn(f"kotflash_amd native module not usable ({exc}); calls take the slower "
+                          "Python launch path. Build it with `python -m kotflash_amd.build`",
+                          RuntimeWarning, stacklevel=2)
+            _native = _NoNative()
         _NATIVE = _native
     return _NATIVE
 

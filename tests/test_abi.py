@@ -44,6 +44,30 @@ def test_library_has_gfx950_code_object_only():
     assert "sm_" not in re.findall(r"amdgcn-amd-amdhsa--(\w+)", out)
 
 
+def test_library_runs_without_the_native_module(monkeypatch):
+    """A native module that does not load (here: not importable) leaves the
+    kernel library usable; every call goes to the Python launch path, and the
+    reason is reported once."""
+    import sys
+    import warnings
+
+    import kotflash_amd
+
+    monkeypatch.setitem(sys.modules, "kotflash_amd._native", None)
+    monkeypatch.delattr(kotflash_amd, "_native", raising=False)
+    monkeypatch.setattr(_hip, "_NATIVE", None)
+    _hip.lib.cache_clear()
+    try:
+        assert _hip.library_available()
+        with pytest.warns(RuntimeWarning, match="native module not usable"):
+            assert _hip.native().attention() is NotImplemented
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            assert _hip.native().store_lengths() is NotImplemented
+    finally:
+        _hip.lib.cache_clear()
+
+
 def _arr(*vals):
     return ctypes.cast((ctypes.c_int64 * len(vals))(*vals), _hip._I64P)
 
