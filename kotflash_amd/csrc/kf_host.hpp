@@ -50,7 +50,8 @@ struct FormCost {
 };
 
 // Fitted to 580 shapes on MI355X (1 to 32 heads, batches of 1 to 16, 45 to
-// 4096 queries, 45 to 6600 keys, up to 1024 tiles; rms error 3 to 14%).
+// 4096 queries, 45 to 6600 keys, up to 1024 tiles; rms error of one form's time
+// 3 to 14%; which of two forms is faster is measured at attn_form).
 constexpr FormCost kFwdCosts[4][kNumForms] = {  // by head-dim tile / 32 - 1; forms as in AttnForm
     {{3.39f, 0.00f, 0.58f, 0.44f, 2}, {0.90f, 2.98f, 0.83f, 0.87f, 1}, {3.38f, 0.28f, 0.59f, 0.46f, 2},
      {1.21f, 2.63f, 0.91f, 0.91f, 1}, {3.08f, 0.72f, 0.46f, 0.45f, 1}, {0, 0, 0, 0, 0}},
@@ -103,20 +104,31 @@ inline float attn_form_cost(const FormCost& c, const FormShape& f, int64_t heads
 // The form of a problem. The default is 1x4 for grids of 128-row tiles that
 // leave most of the 256 CUs idle (at most 64 tiles, 128 when causal, whose
 // tiles differ in length) and 4x1 for the others; another form is taken when
-// the costs above make it at least 8% faster, a margin that covers most of
-// their error. Over the 580 shapes this took the forward 5% and dQ 7% off the
-// default time in the geometric mean (up to 54%: dQ, B=4 H=8 Sq=300 Sk=1500
-// D=128, 58.9 -> 26.8 us); of the 162 that changed form 2 got more than 4%
-// slower (6% at most).
-constexpr int64_t kFormMaxTiles = 512;  // past two 4x1 workgroups per CU other forms lost 5-18%
+// the costs above make it at least 8% faster, up to two 4x1 workgroups per CU.
+//
+// Past one 4x1 workgroup per CU a non-causal grid takes only forms that also
+// keep two on a CU: its tiles are equal, the second workgroup hides the latency
+// that key groups would, and a form alone on its CU adds a round and a merge.
+// The costs do not show that: they price 4x2 up to 15% ahead of 4x1 there, and
+// it measured up to 23% behind (forward, 128 heads, 384 x 4343 D=128 bf16,
+// 128.4 -> 157.6 us; dQ 2x2, 64 heads, 710 x 5854 D=80, 143.6 -> 166.4), while
+// 2x2 at D=64, two per CU, is ahead (forward, 32 heads, 1195 x 3664, 70.1 ->
+// 62.6). Causal tiles differ in length, and more workgroups even them out.
+//
+// Measured with every form over 1884 shapes of up to 640 tiles, against the
+// default form: forward 6.5% and dQ 4.0% faster in the geometric mean; 3
+// forwards got 4 to 8% slower (by 0.3 to 1.1 us) and 10 dQ 4 to 8% (by 0.3 to
+// 0.9 us), most of them with one or two key tiles.
+constexpr int64_t kFormMaxTiles = 512;
 
 inline AttnForm attn_form(const FormCost (&costs)[kNumForms], int64_t heads, int64_t Sq, int64_t Sk, bool causal) {
   const int64_t tiles = (Sq + 127) / 128 * heads;
   if (tiles > kFormMaxTiles) return kForm4x1;
+  const int resident = !causal && tiles > 256 ? 2 : 1;  // least workgroups per CU
   int best = Sk > 128 && tiles <= (causal ? 128 : 64) ? kForm1x4 : kForm4x1;
   float least = 0.92f * attn_form_cost(costs[best], kFormShapes[best], heads, Sq, Sk, causal);
   for (int f = 0; f < kNumForms; ++f) {
-    if (costs[f].per_cu == 0) continue;
+    if (costs[f].per_cu < resident) continue;
     const float t = attn_form_cost(costs[f], kFormShapes[f], heads, Sq, Sk, causal);
     if (t < least) {
       least = t;
@@ -129,9 +141,10 @@ inline AttnForm attn_form(const FormCost (&costs)[kNumForms], int64_t heads, int
 // Whether a causal grid takes its tiles in fold_rank's order: when all its
 // workgroups are resident at once, in more than one per CU, so that the
 // pairing on a CU is decided by the order alone, and the tiles of a head
-// differ enough in length. Measured (tiled form, forward / dQ): B=1 Hq=32
-// Hkv=8 S=1777 D=128 bf16 -6.7% / -4.2%, B=1 Hq=16 S=4096 D=64 dQ -5.8%, four
-// tiles per head (B=8 Hq=12 S=386 D=128) +6%.
+// differ enough in length. Measured over 47 forward and 41 dQ grids of the 4x1
+// form, folded against unfolded, geometric means, forward / dQ: under 8 tiles
+// per head 0.991 / 1.002 (the worst 1.026 and 1.027), 8 to 11 0.981 / 0.969,
+// 12 to 23 0.967 / 0.954, 24 and more 0.967 / 0.940.
 inline int fold_tiles(int64_t tiles_per_head, int64_t grid, int per_cu) {
   return tiles_per_head >= 8 && grid > 256 && grid <= 256 * per_cu;
 }
