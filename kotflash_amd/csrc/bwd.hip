@@ -1504,9 +1504,28 @@ static int launch_dq_form(BwdParams p, bool causal, hipStream_t stream) {
   p.fold = fold_tiles(p.nqt, grid.x, dq_wgs_per_cu(DT, RB, KG));
   if (causal)
     hipLaunchKernelGGL((dq_kernel<T, DT, KS, true, RB, KG>), grid, blk, 0, stream, p);
+  else if constexpr (DT == 128 && RB == 4 && KG == 2)
+    return set_error(KF_EUNSUPPORTED, "kf_attn_bwd: dQ form 4x2 is not built for D > 96 without a mask");
   else
     hipLaunchKernelGGL((dq_kernel<T, DT, KS, false, RB, KG>), grid, blk, 0, stream, p);
   return check_launch("kf_attn_bwd(dq)");
+}
+
+template <typename T, int DT, int KS>
+static int launch_dq(const BwdParams& p, bool causal, hipStream_t stream) {
+  switch (attn_form(kDqCosts[DT / 32 - 1], p.B * p.Hq, p.Sq, p.Sk, causal)) {
+    case kForm4x2: return launch_dq_form<T, DT, KS, 4, 2>(p, causal, stream);
+    case kForm2x2: return launch_dq_form<T, DT, KS, 2, 2>(p, causal, stream);
+    case kForm2x4:
+      if constexpr (form_built(DT, kForm2x4)) return launch_dq_form<T, DT, KS, 2, 4>(p, causal, stream);
+      break;
+    case kForm1x8:
+      if constexpr (form_built(DT, kForm1x8)) return launch_dq_form<T, DT, KS, 1, 8>(p, causal, stream);
+      break;
+    case kForm1x4: return launch_dq_form<T, DT, KS, 1, 4>(p, causal, stream);
+    default: break;
+  }
+  return launch_dq_form<T, DT, KS, 4, 1>(p, causal, stream);
 }
 
 template <typename T, int DT, int KS>
@@ -1520,19 +1539,7 @@ static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) 
     if (rc) return rc;
   }
   if (stages & KF_BWD_DQ) {
-    int rc = KF_OK;
-    switch (attn_form(kDqCosts[DT / 32 - 1], p.B * p.Hq, p.Sq, p.Sk, causal)) {
-      case kForm4x2: rc = launch_dq_form<T, DT, KS, 4, 2>(p, causal, stream); break;
-      case kForm2x2: rc = launch_dq_form<T, DT, KS, 2, 2>(p, causal, stream); break;
-      case kForm2x4:
-        if constexpr (DT <= 64) rc = launch_dq_form<T, DT, KS, 2, 4>(p, causal, stream);
-        break;
-      case kForm1x8:
-        if constexpr (DT == 64) rc = launch_dq_form<T, DT, KS, 1, 8>(p, causal, stream);
-        break;
-      case kForm1x4: rc = launch_dq_form<T, DT, KS, 1, 4>(p, causal, stream); break;
-      default: rc = launch_dq_form<T, DT, KS, 4, 1>(p, causal, stream); break;
-    }
+    const int rc = launch_dq<T, DT, KS>(p, causal, stream);
     if (rc) return rc;
   }
   if (stages & KF_BWD_DKDV) {

@@ -643,10 +643,10 @@ static int launch_fwd(const FwdParams& p, bool causal, hipStream_t stream) {
     case kForm4x2: return launch_fwd_form<T, DT, KS, 4, 2>(p, causal, stream);
     case kForm2x2: return launch_fwd_form<T, DT, KS, 2, 2>(p, causal, stream);
     case kForm2x4:
-      if constexpr (DT <= 64) return launch_fwd_form<T, DT, KS, 2, 4>(p, causal, stream);
+      if constexpr (form_built(DT, kForm2x4)) return launch_fwd_form<T, DT, KS, 2, 4>(p, causal, stream);
       break;
     case kForm1x8:
-      if constexpr (DT == 64) return launch_fwd_form<T, DT, KS, 1, 8>(p, causal, stream);
+      if constexpr (form_built(DT, kForm1x8)) return launch_fwd_form<T, DT, KS, 1, 8>(p, causal, stream);
       break;
     case kForm1x4: return launch_fwd_form<T, DT, KS, 1, 4>(p, causal, stream);
     default: break;

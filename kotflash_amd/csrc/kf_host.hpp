@@ -73,6 +73,20 @@ constexpr FormCost kDqCosts[4][kNumForms] = {  // by head-dim tile / 32 - 1; for
      {0, 0, 0, 0, 0}, {0.95f, 5.68f, 1.59f, 1.77f, 1}, {0, 0, 0, 0, 0}},
 };
 
+// The forms that the kernels are built in, by head-dim tile: exactly the priced
+// ones. (dQ 4x2 at D=128 only causal: without the mask it costs more than 4x1
+// up to 53 key tiles, and more than 0.92 of it beyond.)
+constexpr bool form_built(int head_tile, int form) {
+  return form == kForm2x4 ? head_tile <= 64 : form != kForm1x8 || head_tile == 64;
+}
+constexpr bool priced_forms_are_built(const FormCost (&costs)[4][kNumForms]) {
+  for (int t = 0; t < 4; ++t)
+    for (int f = 0; f < kNumForms; ++f)
+      if ((costs[t][f].per_cu > 0) != form_built(32 * (t + 1), f)) return false;
+  return true;
+}
+static_assert(priced_forms_are_built(kFwdCosts) && priced_forms_are_built(kDqCosts));
+
 inline float attn_form_cost(const FormCost& c, const FormShape& f, int64_t heads, int64_t Sq, int64_t Sk,
                             bool causal) {
   const int rows = 32 * f.rb, keys = 64 * f.kg;

@@ -70,7 +70,9 @@ def test_form_limits(form_of):
     problems = [(kernel, d, heads, sq, sk, causal) for kernel in ("fwd", "dq") for d in (32, 64, 80, 96, 128)
                 for heads in (1, 2, 7, 16, 64, 257, 513) for sq in lengths for sk in lengths
                 for causal in (False, True)]
-    for (_, d, heads, sq, _, causal), form in zip(problems, form_of(problems)):
+    for (kernel, d, heads, sq, _, causal), form in zip(problems, form_of(problems)):
+        # Not built: never priced ahead of 4x1.
+        assert (kernel, d, causal, form) != ("dq", 128, False, "4x2")
         tiles = -(-sq // 128) * heads
         if tiles > 512 or (tiles > 256 and not causal and d > 64):
             assert form == "4x1"
