@@ -78,3 +78,21 @@ def test_form_limits(form_of):
             assert form == "4x1"
         elif tiles > 256 and not causal:
             assert form in ("4x1", "2x2")
+
+
+def test_gpu_shapes_reach_every_form(form_of):
+    """The shapes that tests/test_gpu_forms.py runs reach every form that the
+    rule gives either kernel, at every head-dim tile, causal and not."""
+    from tests.test_gpu_forms import HEAD_DIMS, SHAPES
+
+    def reach(problems):
+        return {(p[0], p[1], p[5], form) for p, form in zip(problems, form_of(problems))}
+
+    kinds = [(kernel, d, causal) for kernel in ("fwd", "dq") for d in HEAD_DIMS for causal in (False, True)]
+    sizes = [int(20 * 1.3 ** i) for i in range(29)]
+    every = reach([(kernel, d, heads, sq, sk, causal) for kernel, d, causal in kinds
+                   for heads in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256)
+                   for sq in sizes for sk in sizes])
+    run = reach([(kernel, d, b * hq, sq, sk, causal) for kernel, d, causal in kinds
+                 for b, hq, _, sq, sk, c in SHAPES if c == causal])
+    assert every - run == set()
