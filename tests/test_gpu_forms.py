@@ -27,7 +27,7 @@ SHAPES = [  # b, hq, hkv, sq, sk, causal
     (1, 1, 1, 23, 29, False), (2, 8, 4, 1715, 2553, False), (2, 16, 4, 283, 270, False),
     (1, 1, 1, 23, 6080, False), (3, 4, 4, 1334, 741, True), (1, 1, 1, 1332, 1437, True),
     (3, 4, 2, 2518, 1099, True), (5, 9, 3, 1030, 1030, True), (2, 3, 3, 5873, 1254, True),
-    (2, 3, 1, 5493, 1280, True),
+    (2, 3, 1, 5493, 1280, True), (1, 4, 2, 4197, 3140, True),
 ]
 
 
