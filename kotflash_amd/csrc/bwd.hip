@@ -33,8 +33,8 @@
 // P and dS are rounded to the input dtype before the products that consume
 // them, as in the reference (:85, :183-184).
 #include <algorithm>
-#include <cstring>
 
+#include "dkdv_plan.hpp"
 #include "kf_common.hpp"
 #include "kf_host.hpp"
 
@@ -75,51 +75,6 @@ struct BwdParams {
   float scale, scale_log2;
 };
 
-// Key-stationary tiling shared by dkdv_kernel, the fixup and the host.
-constexpr int kBNK = 128;  // keys per tile
-constexpr int kBMQ = 64;   // query rows per unit
-
-__host__ __device__ inline int dkdv_qstart(int kt, bool causal) {
-  // Under the upper-left causal mask, query i sees key j iff j <= i, so no
-  // query before the tile's first key (kt * 128) contributes.
-  return causal ? kt * (kBNK / kBMQ) : 0;
-}
-__host__ __device__ inline int dkdv_nq(int kt, int nqt, bool causal) {
-  const int n = nqt - dkdv_qstart(kt, causal);
-  return n > 0 ? n : 0;
-}
-// Key tiles that hold any visible (query, key) pair: all of them, or under
-// the causal mask those before ceil(nqt / 2) (dkdv_nq is zero from there).
-__host__ __device__ inline int dkdv_seen_tiles(int nqt, int nkt, bool causal) {
-  // dkdv_nq(kt) = nqt - 2 kt under the causal mask: zero from ceil(nqt / 2).
-  const int m = causal ? (nqt + 1) / 2 : nkt;
-  return m < nkt ? m : nkt;
-}
-// Order of the key tiles within a KV group: position pos holds tile
-// dkdv_tile_at(pos). The seen tiles alternate from both ends (0, m - 1, 1,
-// m - 2, ...), so that under the causal mask a long tile row is followed by
-// a short one; tiles that see no query come last. With the causal triangle's
-// rows, 256 - 8 kt units at config 3, each pair then costs about two
-// workgroups, and the stream-K boundaries cut every pair once, in its long
-// tile: at most two shares per tile and two segments per workgroup.
-__host__ __device__ inline int dkdv_tile_at(int pos, int m) {
-  if (pos >= m) return pos;
-  return (pos & 1) ? m - 1 - (pos >> 1) : pos >> 1;
-}
-__host__ __device__ inline int dkdv_pos_of(int kt, int m) {
-  if (kt >= m) return kt;
-  return kt < (m + 1) / 2 ? 2 * kt : 2 * (m - 1 - kt) + 1;
-}
-// Stream-K shares: workgroup w owns units [start[w], start[w + 1]). The host
-// places the boundaries by cost rather than by unit count: every key-tile row
-// a workgroup enters (a "segment") costs about kSegmentCost units on top of
-// its units (loading the keys' K/V rows, filling the LDS ring, flushing the
-// accumulators), and the short rows of the causal triangle's far end would
-// otherwise pile many segments onto the last workgroups.
-constexpr int kMaxDkdvWG = 512;
-struct DkdvSplit {
-  int start[kMaxDkdvWG + 1];
-};
 // Units are ordered (KV group, key tile in dkdv_tile_at order, query head,
 // query tile), and the
 // shares are laid out so that XCD x (the dispatcher sends workgroup i to XCD
@@ -1320,13 +1275,6 @@ __global__ __launch_bounds__(256) void dkdv_fixup_kernel(const BwdParams p, cons
   }
 }
 
-// Stream-K bookkeeping from the host: total units and the workgroup count.
-static int64_t dkdv_total_units(int ngroups, int G, int nqt, int nkt, bool causal) {
-  int64_t U = 0;
-  for (int kt = 0; kt < nkt; ++kt) U += (int64_t)ngroups * G * dkdv_nq(kt, nqt, causal);
-  return U;
-}
-
 static int device_cu_count() {
   int dev = 0, n = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 256;
@@ -1341,156 +1289,8 @@ static int dkdv_workgroups() {
   return n < kMaxDkdvWG ? n : kMaxDkdvWG;
 }
 
-// Shares of a problem: one per CU, or fewer where they would hold less than
-// kMinShareUnits units each: a share then costs more in its segment starts and
-// in the fp32 partials that the fixup sums (one per share and row it touches)
-// than its units take. A multiple of 8, for the XCD mapping. Measured over
-// twelve small shapes, us for dK/dV and fixup, one share per CU -> 4 -> 8
-// units: B=1 Hq=8 Hkv=1 S=700 D=96 41.2 -> 33.0 -> 27.4, B=2 Hq=8 Hkv=2 S=1024
-// D=64 causal 28.6 -> 28.4 -> 24.3, B=2 Hq=8 Hkv=2 S=512 D=64 causal 22.9 ->
-// 19.2 -> 20.6; 8 is 4% ahead of 4 in the geometric mean.
-constexpr int kMinShareUnits = 8;
-static int dkdv_share_count(int nwg, int64_t units, int64_t rows) {
-  // Not below one share per tile row: whole rows cost no partials.
-  const int64_t n = ((units / kMinShareUnits > rows ? units / kMinShareUnits : rows) + 7) / 8 * 8;
-  return n < 8 ? (nwg < 8 ? nwg : 8) : n < nwg ? (int)n : nwg;
-}
-
 static size_t delta_bytes(int64_t B, int64_t Hq, int64_t Sq) {
   return ((size_t)B * Hq * Sq * sizeof(float) + 255) / 256 * 256;
-}
-
-// Cost-weighted stream-K boundaries (see DkdvSplit). A segment start costs
-// kSegmentCost8 / 8 units: on the MI355X at config 3 a sweep of the weight
-// put the shortest launch at 4.5 to 6 units, and after a segment's loads
-// came to overlap the previous segment's flush, 3 and 4 units were still
-// 1-2% slower than 5. With the long-short tile order and cuts charged to the
-// share that makes them, 3, 7 and 10 units were 0.4-1.2% slower than 5.
-constexpr int kSegmentCost8 = 40;
-// Cut tile rows also cost their fp32 partials, stored by the dK/dV launch and
-// summed by a fixup launch of its own. Shares of whole consecutive rows cost
-// neither, and are taken when that leaves the longest share no more than this
-// (8ths of a unit, by head-dim tile / 32 - 1) above an even one. Measured, us
-// for dK/dV and fixup, cut -> whole rows: B=4 H=12 S=1000 D=64 causal 41.4 ->
-// 27.9 (longest share 26.1 units against 21.0), B=4 H=16 S=512 D=128 causal
-// 39.4 -> 24.1 (13.0, 10.0), B=4 H=12 S=2048 D=64 causal 90.7 -> 76.7 (81.2,
-// 66.0), B=1 H=8 S=2000 D=128 52.3 -> 64.3 (37.4, 18.5). Over 19 shapes the cuts
-// cost 11 to 31 units at D = 128 and 14 to 32 at D = 64.
-constexpr int kFixupCost8[4] = {112, 112, 104, 88};
-constexpr int kMaxWholeRows = 1024;
-// Returns the number of tile rows that a share boundary cuts (shared tiles).
-// `fixup8`: what cuts cost besides their segment starts (kFixupCost8).
-static int dkdv_split(DkdvSplit& sp, int ngroups, int G, int nqt, int nkt, bool causal, int nwg, int fixup8) {
-  struct Key {
-    int ngroups, G, nqt, nkt, causal, nwg, fixup8;
-  };
-  thread_local Key last{-1, 0, 0, 0, 0, 0, 0};
-  thread_local DkdvSplit cached;
-  thread_local int cached_shared = 0;
-  const Key k{ngroups, G, nqt, nkt, causal ? 1 : 0, nwg, fixup8};
-  if (memcmp(&k, &last, sizeof k) != 0) {
-    int64_t rows_cost = 0, all_units = 0;
-    for (int kt = 0; kt < nkt; ++kt) {
-      const int64_t units = (int64_t)G * dkdv_nq(kt, nqt, causal);
-      if (units) rows_cost += (int64_t)ngroups * (8 * units + kSegmentCost8);
-      all_units += (int64_t)ngroups * units;
-    }
-    const int mseen = dkdv_seen_tiles(nqt, nkt, causal);
-    // Boundaries at equal cost over the rows in unit order (KV group outer,
-    // key tiles in dkdv_tile_at order inner). A boundary inside a tile row
-    // starts one more segment (the next share enters the row part-way); with
-    // cut_cost = kSegmentCost8 that segment start is charged to the share
-    // that makes it, and `total` must then include the cuts. Returns the
-    // number of cuts; `shared` counts the rows cut at least once.
-    auto place = [&](DkdvSplit& out, int64_t total, int64_t cut_cost, int& shared_rows) {
-      int w = 1, cuts = 0;
-      int64_t base = 0, cost = 0;
-      shared_rows = 0;
-      out.start[0] = 0;
-      for (int g = 0; g < ngroups && w < nwg; ++g) {
-        for (int pos = 0; pos < nkt && w < nwg; ++pos) {
-          const int64_t units = (int64_t)G * dkdv_nq(dkdv_tile_at(pos, mseen), nqt, causal);
-          if (!units) continue;
-          const int64_t row_cost = 8 * units + kSegmentCost8;
-          int row_cuts = 0;
-          int64_t prev = 0;  // boundaries never move backwards
-          while (w < nwg) {
-            const int64_t target = (total * w + nwg - 1) / nwg;
-            if (target > cost + row_cost + row_cuts * cut_cost) break;
-            int64_t into = (target - cost - kSegmentCost8 - row_cuts * cut_cost + 7) / 8;
-            into = into < prev ? prev : (into > units ? units : into);
-            prev = into;
-            out.start[w++] = (int)(base + into);
-            if (into > 0 && into < units) ++row_cuts;
-          }
-          shared_rows += row_cuts > 0 ? 1 : 0;
-          cuts += row_cuts;
-          cost += row_cost + row_cuts * cut_cost;
-          base += units;
-        }
-      }
-      while (w < nwg) out.start[w++] = (int)all_units;
-      out.start[nwg] = (int)all_units;
-      return cuts;
-    };
-    // The plain placement first; then the cut-charged one, started from the
-    // plain cut count and kept when it reaches a fixed point (at config 3
-    // at once: the long tile of each pair is cut once, half a segment later).
-    int shared = 0;
-    int cuts = place(cached, rows_cost, 0, shared);
-    DkdvSplit refined;
-    for (int pass = 0; pass < 3; ++pass) {
-      int rshared = 0;
-      const int rcuts = place(refined, rows_cost + (int64_t)cuts * kSegmentCost8, kSegmentCost8, rshared);
-      if (rcuts == cuts) {
-        cached = refined;
-        shared = rshared;
-        break;
-      }
-      cuts = rcuts;
-    }
-    // Shares of whole rows, the longest of them as short as consecutive rows
-    // allow: a bound on a share's cost is feasible if filling shares up to it
-    // needs no more than nwg of them.
-    const int rows = ngroups * mseen;
-    if (shared > 0 && mseen == nkt && rows <= kMaxWholeRows) {
-      auto pack = [&](DkdvSplit& out, int64_t bound) {
-        int w = 0;
-        int64_t base = 0, in = 0;
-        out.start[0] = 0;
-        for (int g = 0; g < ngroups; ++g)
-          for (int pos = 0; pos < nkt; ++pos) {
-            const int64_t units = (int64_t)G * dkdv_nq(dkdv_tile_at(pos, mseen), nqt, causal);
-            const int64_t c = 8 * units + kSegmentCost8;
-            if (c > bound) return false;
-            if (in + c > bound) {
-              if (++w == nwg) return false;
-              out.start[w] = (int)base;
-              in = 0;
-            }
-            in += c;
-            base += units;
-          }
-        while (++w <= nwg) out.start[w] = (int)all_units;
-        return true;
-      };
-      int64_t lo = rows_cost / nwg, hi = lo + fixup8;
-      DkdvSplit whole;
-      if (pack(whole, hi)) {
-        shared = 0;
-        while (hi - lo > 8) {
-          cached = whole;
-          const int64_t mid = (lo + hi) / 2;
-          if (pack(whole, mid)) hi = mid; else { lo = mid; whole = cached; }
-        }
-        cached = whole;
-      }
-    }
-    cached_shared = shared;
-    last = k;
-  }
-  sp = cached;
-  return cached_shared;
 }
 
 static size_t partial_bytes(int nwg, int64_t D) {
@@ -1542,36 +1342,30 @@ static int launch_bwd(BwdParams p, bool causal, int stages, hipStream_t stream) 
     const int rc = launch_dq<T, DT, KS>(p, causal, stream);
     if (rc) return rc;
   }
+  if (!(stages & (KF_BWD_DKDV | KF_BWD_DKDV_FIXUP))) return KF_OK;
+  p.nqt = cdiv(p.Sq, kBMQ);
+  p.nkt = cdiv(p.Sk, kBNK);
+  p.units = dkdv_total_units(p.ngroups, p.G, p.nqt, p.nkt, causal);
+  if (p.units > 0x7fffffff) return set_error(KF_EINVAL, "kf_attn_bwd: problem too large for one dK/dV launch");
+  const DkdvPlan& plan = dkdv_plan(p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg, kFixupCost8[DT / 32 - 1]);
+  p.nwg = plan.nwg;
   if (stages & KF_BWD_DKDV) {
-    p.nqt = cdiv(p.Sq, kBMQ);
-    p.nkt = cdiv(p.Sk, kBNK);
-    p.units = dkdv_total_units(p.ngroups, p.G, p.nqt, p.nkt, causal);
-    p.nwg = dkdv_share_count(p.nwg, p.units, (int64_t)p.ngroups * dkdv_seen_tiles(p.nqt, p.nkt, causal));
-    if (p.units > 0x7fffffff) return set_error(KF_EINVAL, "kf_attn_bwd: problem too large for one dK/dV launch");
-    DkdvSplit sp;
-    dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg, kFixupCost8[DT / 32 - 1]);
     if (causal)
-      hipLaunchKernelGGL((dkdv_kernel<T, DT, KS, true>), dim3((unsigned)p.nwg), dim3(256), 0, stream, p, sp);
+      hipLaunchKernelGGL((dkdv_kernel<T, DT, KS, true>), dim3((unsigned)p.nwg), dim3(256), 0, stream, p, plan.split);
     else
-      hipLaunchKernelGGL((dkdv_kernel<T, DT, KS, false>), dim3((unsigned)p.nwg), dim3(256), 0, stream, p, sp);
+      hipLaunchKernelGGL((dkdv_kernel<T, DT, KS, false>), dim3((unsigned)p.nwg), dim3(256), 0, stream, p, plan.split);
     int rc = check_launch("kf_attn_bwd(dkdv)");
     if (rc) return rc;
   }
   if (stages & KF_BWD_DKDV_FIXUP) {
-    p.nqt = cdiv(p.Sq, kBMQ);
-    p.nkt = cdiv(p.Sk, kBNK);
-    p.units = dkdv_total_units(p.ngroups, p.G, p.nqt, p.nkt, causal);
-    p.nwg = dkdv_share_count(p.nwg, p.units, (int64_t)p.ngroups * dkdv_seen_tiles(p.nqt, p.nkt, causal));
-    DkdvSplit sp;
-    const int shared = dkdv_split(sp, p.ngroups, p.G, p.nqt, p.nkt, causal, p.nwg, kFixupCost8[DT / 32 - 1]);
     const int64_t unseen = (int64_t)p.ngroups * (p.nkt - dkdv_seen_tiles(p.nqt, p.nkt, causal));
-    if (shared > 0 || unseen > 0) {
+    if (plan.shared > 0 || unseen > 0) {
       const int64_t grid = (int64_t)p.nkt * p.ngroups * kFixSub;
       if (grid > 0x7fffffff) return set_error(KF_EINVAL, "kf_attn_bwd: problem too large for one fixup launch");
       if (causal)
-        hipLaunchKernelGGL((dkdv_fixup_kernel<T, DT, true>), dim3((unsigned)grid), dim3(256), 0, stream, p, sp);
+        hipLaunchKernelGGL((dkdv_fixup_kernel<T, DT, true>), dim3((unsigned)grid), dim3(256), 0, stream, p, plan.split);
       else
-        hipLaunchKernelGGL((dkdv_fixup_kernel<T, DT, false>), dim3((unsigned)grid), dim3(256), 0, stream, p, sp);
+        hipLaunchKernelGGL((dkdv_fixup_kernel<T, DT, false>), dim3((unsigned)grid), dim3(256), 0, stream, p, plan.split);
       int rc = check_launch("kf_attn_bwd(dkdv fixup)");
       if (rc) return rc;
     }
