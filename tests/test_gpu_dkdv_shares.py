@@ -1,8 +1,9 @@
 """dK/dV at the edges of its share plans: shares of whole tile rows (with and
 without room to spare), rows cut into many shares (the fixup's batches of four
-and their remainders), fewer shares than CUs, a single unit, and keys that no
-query sees. Against float32 autograd at the backward's fp16 bar; dK/dV sum up
-to 8 heads of a group, so the outputs are scaled to a few units at most."""
+and their remainders) or into few (whose shares are shorter), fewer shares than
+CUs, a single unit, and keys that no query sees. Against float32 autograd at the
+backward's fp16 bar; dK/dV sum up to 8 heads of a group, so the outputs are
+scaled to a few units at most."""
 import math
 
 import pytest
@@ -22,6 +23,7 @@ F16 = torch.float16
     (1, 8, 1, 700, 700, False), (1, 8, 1, 700, 700, True), (2, 8, 2, 1024, 1024, True),
     (1, 1, 1, 1, 1, True), (1, 1, 1, 64, 129, False), (2, 4, 1, 200, 900, True),
     (1, 32, 4, 500, 500, True), (8, 12, 12, 1024, 1024, True),
+    (3, 16, 8, 533, 533, True), (1, 16, 4, 433, 433, True), (3, 8, 1, 88, 2355, False),
 ], ids=str)
 def test_dkdv_share_plans(shape, d):
     b, hq, hkv, sq, sk, causal = shape

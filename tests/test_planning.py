@@ -152,7 +152,7 @@ def test_gfx950_envelope():
 
 
 def test_gfx950_auto_routing_by_size():
-    """auto keeps host-bound small problems on SDPA, takes the HIP kernels
+    """auto keeps small training problems on SDPA, takes the HIP kernels
     from about 1.5e9 forward FLOP up, and always for split-KV decode."""
     f16 = dict(dtype_name="float16")
     # Config 1: 4 * 64 * 16 * 131328 (the survey's algorithmic work figure).
