@@ -106,18 +106,18 @@ def gfx950_decode_eligible(sq: int, sk: int, d: int, *, causal: bool) -> bool:
             and gfx950_head_dim_ok(d))
 
 
-# Below this much forward work (FLOP) an eager training call (forward, then
-# backward through autograd) is bound by host time, and PyTorch's SDPA,
-# whose launch and autograd paths are C++, finishes first. Measured on MI355X
-# through the public API (python -m kotflash_amd.benchmark, B=2 Hq=8 Hkv=2
-# D=64 causal, fp16; fwd+bwd us, HIP vs SDPA):
-#   S=256: 220 vs 183;  S=512: 216 vs 179;  S=1024: 213 vs 262;
-#   S=2048: 261 vs 411 (an earlier run);  B=1 H=8 S=512 D=128 non-causal
-#   (1.1e9 FLOP): 215 vs 174.
-# Inference calls (no backward to follow) are not subject to it: the HIP
-# forward's launch path is the shorter one (config 1, S=512: 18.9 us per call
-# against 22.4 us for SDPA, bench.py torch_sdpa_same_gpu), and split-KV decode
-# shapes are 22x faster (config 2).
+# Training calls (forward, then backward through autograd) below this much
+# forward work (FLOP) go to PyTorch's SDPA. The line dates from a Python launch
+# path whose host time bounded a small step (fwd+bwd 213-220 us, where SDPA took
+# 179 us at S=512 and 262 at S=1024, B=2 Hq=8 Hkv=2 D=64 causal). Through the
+# C++ launch path the HIP step is ahead on both sides of it, measured on MI355X
+# through the public API, fp16 (fwd+bwd us, HIP / SDPA): B=1 H=4 S=64 D=64 causal
+# (2.1e6 FLOP) 71 / 98; B=2 Hq=8 Hkv=2 D=64 causal S=256 71 / 108, S=512 73 / 124,
+# S=1024 74 / 227, S=2048 91 / 371; B=1 H=8 S=512 D=128 non-causal (1.1e9 FLOP)
+# 67 / 108. The line is unchanged: backend="hip" takes the kernels at any size.
+# Inference calls (no backward to follow) are not subject to it: S=512 takes
+# 5.8 us per call against 22.4 for SDPA, and split-KV decode shapes are over 20
+# times faster.
 GFX950_HIP_MIN_FWD_FLOPS = 1.5e9
 
 

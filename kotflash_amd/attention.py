@@ -260,9 +260,8 @@ def attention(
     (padded ``PreallocatedKVCache`` views included) with split-KV decode; the
     caller must pass only keys visible to every query. On gfx950, auto uses
     the HIP kernels for fp16/bf16 inference calls and decode shapes, and for
-    training calls (autograd) of at least 1.5e9 forward FLOP, below which an
-    eager training step is host-bound and SDPA finishes first; SDPA
-    everywhere else.
+    training calls (autograd) of at least 1.5e9 forward FLOP; smaller training
+    calls, and everything else, go to SDPA.
     """
     # The ordinary GPU call is checked, routed and launched natively; anything
     # else (and every error) takes the checks below.

@@ -365,10 +365,14 @@ __global__ __launch_bounds__(64 * RB * KG, dq_waves_per_simd(DT, RB, KG)) void d
   // Where a tile's body issues the next tile's loads: first, or (LATE) after
   // its own first operand reads. A tile whose first key block lies above all
   // of a wave's rows is its group's last, so a late wave misses no load.
-  // Measured, tiled form: after the reads the 64-wide tile runs 1.2-1.9%
-  // faster causal (B=2 Hq=16 Hkv=4 S=4096) and level non-causal, and the
-  // causal 128-wide one 4.3% in bf16 (174.5 against 181.9 us there) but 2%
-  // slower in fp16; the others are level or up to 1% slower.
+  // Measured, tiled form, more than 512 tiles, late against first: the causal
+  // 64-wide tile 0.995 in the geometric mean (41 shapes, 0.963 to 1.023). The
+  // causal 128-wide one in bf16 is even in the mean (28 shapes, 0.998) but not
+  // shape by shape: 1 to 6% ahead at 830 to 1060 tiles (B=2 Hq=16 Hkv=4 S=4096
+  // 179.2 against 187.3 us), up to 9% behind with many short ones (B=16 Hq=16
+  // S=1336 D=112 230 against 210). Late, it runs within 3% of the kernel as it
+  // was before it took forms, on every one of them; no better split is known.
+  // In fp16 it was 2% slower late; the others are level or up to 1% slower.
   constexpr bool LATE = KG == 1 && CAUSAL && (DT == 64 || (DT == 128 && std::is_same_v<T, __bf16>));
   auto tile_body = [&](int li, auto stc) {
     constexpr int ST = decltype(stc)::value;

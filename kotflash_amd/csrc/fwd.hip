@@ -282,10 +282,12 @@ __global__ __launch_bounds__(64 * RB * KG, fwd_waves_per_simd(DT, RB, KG)) void 
 
   // Where a tile's body issues the next tile's loads. The tiled form at head
   // dims above 64 does it behind the S product, whose operand reads they hold
-  // up otherwise (causal B=2 Hq=16 Hkv=4 S=4096 D=128 bf16 133.5 -> 127.9 us,
-  // D=96 -3%, non-causal within 1%). Narrower tiles and the other forms load
-  // first: their shorter steps leave later loads too little time to land (+2
-  // to +4%).
+  // up otherwise (causal B=2 Hq=16 Hkv=4 S=4096 D=128 bf16 139.6 -> 132.0 us).
+  // Geometric means over grids of more than 512 tiles, late against first:
+  // causal 128-wide bf16 0.962 and fp16 0.970 (53 shapes, 0.90 to 1.02), the
+  // 96-wide tile 0.993 (91 shapes) and 128-wide without the mask 0.995 (31).
+  // Narrower tiles and the other forms load first: their shorter steps leave
+  // later loads too little time to land (+2 to +4%).
   constexpr bool LATE = KG == 1 && DT > 64;
   // This wave's li-th tile on ring stage ST (a compile-time constant, so
   // every LDS offset in the body is an immediate).

@@ -16,8 +16,8 @@
 //   causal forward, S=512, same heads                                 15.5 -> 5.8
 //   training step, B=4 H=12 S=1000 D=64 causal                       139.3 -> 79.6
 //   training step, B=4 H=8 Sq=300 Sk=1500 D=80                       129.1 -> 75.1
-// (the two training steps with the backward kernels of that measurement; 65.1
-// and 63.3 with the present forms and dK/dV shares).
+// (the two training steps with the backward kernels of that measurement; 65.9
+// and 59.5 with the present forms and dK/dV plans).
 // The calls are then bound by their kernels and launches (about 2.7 us of host
 // time per launch in this HIP runtime).
 #include <torch/csrc/Exceptions.h>
